@@ -265,3 +265,38 @@ def test_fp8_argument_errors(gpu):
         mla_decode(q8.to(gpu), c8.to(gpu), l8.to(gpu), b8.to(gpu), kv_scale=s8.to(gpu))
     with pytest.raises(AssertionError):
         mla_decode(q.to(gpu), codes.to(gpu), lens.to(gpu), bt.to(gpu), kv_scale=scale[:1].repeat(3).to(gpu))
+
+
+@pytest.mark.parametrize("heads,dtype", [(20, torch.bfloat16), (40, torch.bfloat16), (64, torch.bfloat16),
+                                         (64, torch.float16), (128, torch.bfloat16)])
+def test_late_reference_max_move(gpu, heads, dtype):
+    """Scores of a wide spread (softmax scale 1/4: a standard deviation of 6)
+    move the reference max in later sub-tiles of most heads, so every wave
+    rescales its accumulators by the published factors: with 288 workers along
+    the sequences, workgroups of one, two and four head blocks, whose waves
+    past the head blocks (fewer than four) run the value products only.
+    Budget: probabilities rounded to the element type (half an ulp, at most
+    u = 2^-8 of the value in bf16, 2^-11 in fp16), the partials likewise, and
+    the final half ulp at the largest magnitude the value before it can have;
+    2^-12 for the float32 scores."""
+    from triton_mla import mla_decode
+
+    lens = [2784, 518, 4294]
+    print(f"late max heads={heads} {dtype}", flush=True)
+    q, codes, scale, lens_t, bt = _make(3, heads, lens, dtype=dtype, seed=heads)
+    name, mant, u = ("bf16", 7, 2.0 ** -8) if dtype == torch.bfloat16 else ("fp16", 10, 2.0 ** -11)
+    exact, ref_lse = _oracle(q, codes, scale, lens_t, bt, 0.25, name)
+    A, V = _amag(q, codes, scale, lens_t, bt, 0.25, name)
+    before = (u + 2.0 ** -12) * A + u * V
+    ulp = 2.0 ** (np.floor(np.log2(np.abs(exact) + before)) - mant)
+    # short pieces (rows of one batch), then long ones (the batch 32 times)
+    for copies, splits in ((1, 96), (32, 3)):
+        out, lse = mla_decode(q.to(gpu).repeat(copies, 1, 1), codes.to(gpu), lens_t.to(gpu).repeat(copies),
+                              bt.to(gpu).repeat(copies, 1), softmax_scale=0.25, kv_scale=scale.to(gpu),
+                              num_splits=splits, return_lse=True)
+        torch.cuda.synchronize()
+        err = np.abs(out[:3].double().cpu().numpy() - exact)
+        print(f"splits {splits}: max err / budget {(err / (before + 0.5 * ulp)).max():.3f}", flush=True)
+        assert np.all(err <= before + 0.5 * ulp)
+        np.testing.assert_allclose(lse[:3].cpu().numpy(), ref_lse, rtol=1e-5, atol=1e-5)
+        assert torch.equal(out.view(copies, -1), out[:3].reshape(1, -1).expand(copies, -1))

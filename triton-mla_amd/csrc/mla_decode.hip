@@ -1112,6 +1112,8 @@ void mla_partial_kernel(PartialArgs a) {
         next_page = i < 0 ? pro_page[kStages - 1] : page_fetch(st0 + i + kStages);
       if (F8 && do_copy) sc3 = s_load_f32(a.kv_scale + (int64_t)page * a.sc_s0);  // sub-tile i+3
       const int pbuf = i & 1;
+      // the factors of PV(i) (waves without S read them again where they use
+      // them, see pass1_hook)
       f32x4 alpha4 = ds_read_f32x4(lds + OFF_A + pbuf * ASLOT + (lane & 31) * 16);
       // ring entries (i + 1 >= 0): S(i+1) reads entry i+1, PV(i) entry i
       // (entry 0 at i = -1, where P = 0), the copies fill entry i+3 (16-bit
@@ -1132,8 +1134,7 @@ void mla_partial_kernel(PartialArgs a) {
       // pass 1: S(i+1) and PV(i) steps [0, PV_SPLIT) from step PV_START on;
       // the copies of sub-tile i+3 are spread evenly over the pass's steps,
       // and the factors published for PV(i) are applied before its first
-      // MFMA (the wait of step PV_START - 1 covers their read, which is older
-      // than every read of the pass)
+      // MFMA
       const char* csrc[RG_PER_WAVE];
       auto pass1_hook = [&](auto NSTEPSC) __attribute__((always_inline)) {
         return [&](auto J) __attribute__((always_inline)) {
@@ -1141,7 +1142,16 @@ void mla_partial_kernel(PartialArgs a) {
           constexpr int NST = decltype(NSTEPSC)::value;
           if constexpr (j == 0 && do_copy && !F8) copy_src(st0 + i + kStages - 1, page, csrc);
           if constexpr (j == PV_START - 1) {
-            pin_f4(alpha4);
+            // An S wave's operand waits cover the factors' read, which is
+            // older than every read of the pass. A wave without S has waited
+            // for nothing yet, and its branch may copy registers of a read in
+            // flight: it reads them here and waits.
+            if constexpr (NST == NKC) {
+              pin_f4(alpha4);
+            } else {
+              alpha4 = ds_read_f32x4(lds + OFF_A + pbuf * ASLOT + (lane & 31) * 16);
+              lgkm_tie_f4<0>(alpha4);
+            }
             bool any = false;
 #pragma unroll
             for (int hb = 0; hb < NHB; ++hb) any |= alpha4[hb] != 1.0f;
