@@ -129,6 +129,23 @@ __device__ __forceinline__ void store_through_f32(float* p, float v) {
   asm volatile("global_store_dword %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
 }
 
+// Inclusive sum over the lanes of a wave by DPP moves (rows of 16, then row
+// broadcasts): about ten VALU instructions, where shuffles take six LDS round
+// trips, each on the path of every kernel's start.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int x) {
+  return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan(int x) {
+  x = dpp_add<0x111, 0xF>(x);  // row_shr 1, 2, 4, 8
+  x = dpp_add<0x112, 0xF>(x);
+  x = dpp_add<0x114, 0xF>(x);
+  x = dpp_add<0x118, 0xF>(x);
+  x = dpp_add<0x142, 0xA>(x);  // row_bcast 15 into rows 1 and 3
+  return dpp_add<0x143, 0xC>(x);  // row_bcast 31 into rows 2 and 3
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+
 // POW2: the page size is known to be a power of two (page_shift >= 0)
 template <bool POW2 = false>
 __device__ __forceinline__ int page_slot_of(const PartialArgs& a, int t) {
@@ -168,10 +185,23 @@ struct WorkRange {
   bool snapped;
 };
 
+// Lengths of the sequences as the partition sees them: as given, or cut to
+// what the cache can hold.
+struct GivenLens {
+  const int32_t* seqlens;
+  __device__ __forceinline__ int operator()(int b) const { return seqlens[b]; }
+};
+struct CappedLens {
+  const int32_t* seqlens;
+  int32_t cap;
+  __device__ __forceinline__ int operator()(int b) const { return min(seqlens[b], cap); }
+};
+
 // Returns false when the worker has no tiles (balanced mode only). Every
 // wave computes the same range on its own (registers and cross-lane moves
 // only, no LDS or barrier).
-__device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, WorkRange& w) {
+template <class Lens>
+__device__ __forceinline__ bool work_range(const PartialArgs& a, const Lens& len_of, int worker, WorkRange& w) {
   w.chunk = 0;
   w.seg_cost = 0;
   w.snapped = false;
@@ -180,7 +210,7 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
     // tiles (kernel.py:83-86); worker b * S + s takes piece s
     const int S = a.num_splits;
     const int b = worker / S, s = worker - b * S;
-    w.n_first = a.seqlens[b];
+    w.n_first = len_of(b);
     const int nt = tiles_of(w.n_first);
     const int spt = (nt + S - 1) / S;
     w.tile_lo = s * spt;
@@ -198,23 +228,15 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
   const int lane0 = lane_id_fresh();
   const int per = (a.batch + 63) >> 6;
   const int lo_b = min(lane0 * per, a.batch), hi_b = min(lo_b + per, a.batch);
-  const int len0 = lo_b < hi_b ? a.seqlens[lo_b] : 0;
+  const int len0 = lo_b < hi_b ? len_of(lo_b) : 0;
   int sum = tiles_of(len0), live = len0 > 0;
   for (int b = lo_b + 1; b < hi_b; ++b) {
-    const int nt = tiles_of(a.seqlens[b]);
+    const int nt = tiles_of(len_of(b));
     sum += nt;
     live += nt > 0;
   }
-  int incl = sum;
-  int vsum = sum + kSegCostTiles * live, vincl = vsum;  // positions on the straddling line
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int v = __shfl_up(incl, d), vv = __shfl_up(vincl, d);
-    if (lane0 >= d) {
-      incl += v;
-      vincl += vv;
-    }
-  }
+  const int incl = wave_scan(sum);
+  const int vsum = sum + kSegCostTiles * live, vincl = wave_scan(vsum);  // positions on the straddling line
   const int total = __builtin_amdgcn_readlane(incl, 63);
   const int chunk = (total + a.num_workers - 1) / a.num_workers;
   w.chunk = chunk;
@@ -227,13 +249,8 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
   bool snapped = false;
   if (chunk > 0) {
     pcs = (tiles_of(len0) + chunk - 1) / chunk;  // len0 = 0 for a lane without sequences
-    for (int b = lo_b + 1; b < hi_b; ++b) pcs += (tiles_of(a.seqlens[b]) + chunk - 1) / chunk;
-    pinc = pcs;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(pinc, d);
-      if (lane0 >= d) pinc += v;
-    }
+    for (int b = lo_b + 1; b < hi_b; ++b) pcs += (tiles_of(len_of(b)) + chunk - 1) / chunk;
+    pinc = wave_scan(pcs);
     snapped = __builtin_amdgcn_readlane(pinc, 63) <= a.num_workers;
   }
   w.snapped = snapped;
@@ -241,7 +258,7 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
     // the one lane whose sequences hold piece `worker` finds which of them
     int poff = pinc - pcs, off = incl - sum, fb = lo_b, flen = len0;
     for (int b = lo_b; b < hi_b; ++b) {
-      const int len = b == lo_b ? len0 : a.seqlens[b];
+      const int len = b == lo_b ? len0 : len_of(b);
       const int nt = tiles_of(len);
       const int np = (nt + chunk - 1) / chunk;
       fb = b;
@@ -276,7 +293,7 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
   // the one lane whose sequences hold position vlo finds which of them it is
   int voff = vincl - vsum, fb = lo_b, flen = len0;
   for (int b = lo_b; b < hi_b; ++b) {
-    const int len = b == lo_b ? len0 : a.seqlens[b];
+    const int len = b == lo_b ? len0 : len_of(b);
     const int nt = tiles_of(len);
     const int vt = nt > 0 ? nt + kSegCostTiles : 0;
     fb = b;
@@ -293,6 +310,10 @@ __device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, Wor
   w.tile_lo = max(vlo - w.off_first, 0);
   w.tile_hi = min(vlo + vchunk, vtotal) - w.off_first;
   return true;
+}
+
+__device__ __forceinline__ bool work_range(const PartialArgs& a, int worker, WorkRange& w) {
+  return work_range(a, GivenLens{a.seqlens}, worker, w);
 }
 
 // Where the result of one segment (tiles [t_start, ...) of sequence b, which
@@ -329,6 +350,60 @@ __device__ __forceinline__ SegmentSlot segment_slot(const PartialArgs& a, const 
   }
   s.direct = s.count == 1;
   return s;
+}
+
+// The partial slots of sequence b, slot0 .. slot0 + count - 1 (count 0: an
+// empty sequence, 1: stage 1 wrote the output itself), from the lengths as
+// work_range reads them. Every wave computes them on its own.
+template <class Lens>
+__device__ __forceinline__ void sequence_slots(const Lens& len_of, int batch, int num_splits, int num_workers, int b,
+                                               int& slot0, int& count) {
+  const int lane = threadIdx.x & 63;
+  const int nt_b = tiles_of(len_of(b));
+  slot0 = 0;
+  count = 0;
+  if (num_splits > 0) {
+    const int S = num_splits;
+    if (nt_b > 0) {
+      const int spt = (nt_b + S - 1) / S;
+      count = (nt_b + spt - 1) / spt;
+    }
+    slot0 = b * S;
+    return;
+  }
+  // tiles in all (the snapped form), and positions before b and in all on
+  // the straddling form's line, where every non-empty sequence starts with
+  // kSegCostTiles extra positions (work_range)
+  const int nt0 = lane < batch ? tiles_of(len_of(lane)) : 0;  // this lane's first sequence
+  const int vt0 = nt0 > 0 ? nt0 + kSegCostTiles : 0;
+  int total = nt0, vtotal = vt0, vbefore = lane < b ? vt0 : 0;
+  for (int i = lane + 64; i < batch; i += 64) {
+    const int nt = tiles_of(len_of(i));
+    const int vt = nt > 0 ? nt + kSegCostTiles : 0;
+    total += nt;
+    vtotal += vt;
+    if (i < b) vbefore += vt;
+  }
+  if (nt_b == 0) return;
+  total = wave_total(total);  // > 0
+  const int chunk = (total + num_workers - 1) / num_workers;
+  // the partial kernel's snapped ranges when the pieces fit the workers
+  int ptotal = (nt0 + chunk - 1) / chunk, pbefore = lane < b ? ptotal : 0;
+  for (int i = lane + 64; i < batch; i += 64) {
+    const int np = (tiles_of(len_of(i)) + chunk - 1) / chunk;
+    ptotal += np;
+    if (i < b) pbefore += np;
+  }
+  if (wave_total(ptotal) <= num_workers) {
+    count = (nt_b + chunk - 1) / chunk;
+    slot0 = wave_total(pbefore) + b;
+  } else {  // straddling: the workers whose ranges hold b's tiles
+    const int vchunk = (wave_total(vtotal) + num_workers - 1) / num_workers;
+    const int first = wave_total(vbefore) + kSegCostTiles;  // position of b's tile 0
+    const int g1 = first / vchunk, g2 = (first + nt_b - 1) / vchunk;
+    count = g2 - g1 + 1;
+    slot0 = g1 + b;
+  }
 }
 
 // Stage 1 over an fp8 cache (mla_decode_fp8.hip): grid = (workers, head

@@ -2140,78 +2140,9 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(CombineArgs a) {
   const int b = blockIdx.x;
   const int h_lo = blockIdx.y * 4 * HPW;
   const int h_hi = min(h_lo + 4 * HPW, a.num_heads);
-  __shared__ int s_red[3][4];
 
-  // partial slots of sequence b
-  const int n_b = a.seqlens[b];
-  const int nt_b = tiles_of(n_b);
-  int slot0 = 0, count = 0;
-  if (a.num_splits > 0) {
-    const int S = a.num_splits;
-    if (nt_b > 0) {
-      const int spt = (nt_b + S - 1) / S;
-      count = (nt_b + spt - 1) / spt;
-    }
-    slot0 = b * S;
-  } else {
-    // tiles in all (the snapped form), and positions before b and in all on
-    // the straddling form's line, where every non-empty sequence starts with
-    // kSegCostTiles extra positions (work_range)
-    int total = 0, vbefore = 0, vtotal = 0;
-    for (int i = threadIdx.x; i < a.batch; i += 256) {
-      const int nt = tiles_of(a.seqlens[i]);
-      const int vt = nt > 0 ? nt + kSegCostTiles : 0;
-      total += nt;
-      vtotal += vt;
-      if (i < b) vbefore += vt;
-    }
-    for (int d = 32; d >= 1; d >>= 1) {
-      total += __shfl_xor(total, d);
-      vbefore += __shfl_xor(vbefore, d);
-      vtotal += __shfl_xor(vtotal, d);
-    }
-    if (lane == 0) {
-      s_red[0][wave] = total;
-      s_red[1][wave] = vbefore;
-      s_red[2][wave] = vtotal;
-    }
-    __syncthreads();
-    total = s_red[0][0] + s_red[0][1] + s_red[0][2] + s_red[0][3];
-    vbefore = s_red[1][0] + s_red[1][1] + s_red[1][2] + s_red[1][3];
-    vtotal = s_red[2][0] + s_red[2][1] + s_red[2][2] + s_red[2][3];
-    if (nt_b > 0) {  // (then total > 0; uniform over the workgroup)
-      const int chunk = (total + a.num_workers - 1) / a.num_workers;
-      // the partial kernel's snapped ranges when the pieces fit the workers
-      int pbefore = 0, ptotal = 0;
-      for (int i = threadIdx.x; i < a.batch; i += 256) {
-        const int np = (tiles_of(a.seqlens[i]) + chunk - 1) / chunk;
-        ptotal += np;
-        if (i < b) pbefore += np;
-      }
-      for (int d = 32; d >= 1; d >>= 1) {
-        pbefore += __shfl_xor(pbefore, d);
-        ptotal += __shfl_xor(ptotal, d);
-      }
-      __syncthreads();  // every wave has read s_red
-      if (lane == 0) {
-        s_red[0][wave] = pbefore;
-        s_red[1][wave] = ptotal;
-      }
-      __syncthreads();
-      pbefore = s_red[0][0] + s_red[0][1] + s_red[0][2] + s_red[0][3];
-      ptotal = s_red[1][0] + s_red[1][1] + s_red[1][2] + s_red[1][3];
-      if (ptotal <= a.num_workers) {
-        count = (nt_b + chunk - 1) / chunk;
-        slot0 = pbefore + b;
-      } else {  // straddling: the workers whose ranges hold b's tiles
-        const int vchunk = (vtotal + a.num_workers - 1) / a.num_workers;
-        const int first = vbefore + kSegCostTiles;  // position of b's tile 0
-        const int g1 = first / vchunk, g2 = (first + nt_b - 1) / vchunk;
-        count = g2 - g1 + 1;
-        slot0 = g1 + b;
-      }
-    }
-  }
+  int slot0, count;
+  sequence_slots(GivenLens{a.seqlens}, a.batch, a.num_splits, a.num_workers, b, slot0, count);
   if (count == 1) return;  // written by stage 1
   static_assert(DV == 512, "one row = 64 lanes x 8 elements");
   const MergeView mv{a.mid_o, a.mid_lse, a.num_heads, a.out, a.out_sb, a.out_sh, a.lse};
