@@ -303,10 +303,13 @@ int tmla_mla_decode_fp8_partial(const void* q, int64_t q_stride_b, int64_t q_str
  * log-sum-exp (kernel.py:43-138, launch kernel.py:276-302), which a second
  * kernel merges (kernel.py:141-181, launch kernel.py:303-320). Scores and
  * sums in float32, probabilities rounded to dtype for the value product
- * (kernel.py:123). bf16 / fp16 calls with head_dim_v <= 512 and
- * head_dim_v + rope_dim <= 576 run on matrix cores (v_mfma_f32_16x16x32,
- * 64 heads per workgroup), the others on the vector ALU (16 heads per
- * workgroup): for unusual dims, not at the speed of the kernels above. Arguments mean what they mean for tmla_mla_decode;
+ * (kernel.py:123). bf16 / fp16 calls with head_dim_v in {64, 128, 256, 512},
+ * rope_dim in {16, 32, 64} and 16-byte aligned q, kv and out rows run the
+ * kernels of tmla_mla_decode_generic_balanced; other bf16 / fp16 calls with
+ * head_dim_v <= 512 and head_dim_v + rope_dim <= 576 run on matrix cores too
+ * (v_mfma_f32_16x16x32, 64 heads per workgroup), the others on the vector ALU
+ * (16 heads per workgroup): for unusual dims, not at the speed of the kernels
+ * above. Arguments mean what they mean for tmla_mla_decode;
  * num_splits in [1, 65535]; batch and num_heads at most 65535; the
  * workspace is tmla_generic_workspace_bytes(batch, num_heads, head_dim_v,
  * num_splits) bytes and needs no initialisation. Sequence lengths above the
@@ -328,6 +331,29 @@ int tmla_mla_decode_generic(const void* q, int64_t q_stride_b, int64_t q_stride_
                             int32_t rope_dim, int32_t dtype, float softmax_scale, int32_t num_splits, void* out,
                             int64_t out_stride_b, int64_t out_stride_h, float* lse, void* workspace,
                             size_t workspace_bytes, void* stream);
+
+/*
+ * The same decode with the balanced partition of tmla_mla_decode's
+ * num_splits = 0: the 64-token tiles of all sequences are spread over
+ * num_workers ranges (computed on the device), for head_dim_v in {64, 128,
+ * 256, 512}, rope_dim in {16, 32, 64} and q, kv and out rows on 16-byte
+ * boundaries (TMLA_ERR_UNSUPPORTED otherwise). tmla_generic_workers gives the
+ * worker count that fills a device of `cus` compute units (0: dims the form
+ * does not take); num_workers in [1, 65535]; the workspace is
+ * tmla_generic_balanced_workspace_bytes(batch, num_heads, head_dim_v,
+ * num_workers) bytes, 16-byte aligned, no initialisation. No counterpart in
+ * the reference (its splits are uniform, kernel.py:83-86).
+ */
+int32_t tmla_generic_workers(int32_t head_dim_v, int32_t rope_dim, int32_t dtype, int32_t num_heads, int32_t cus);
+size_t tmla_generic_balanced_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim_v,
+                                             int32_t num_workers);
+int tmla_mla_decode_generic_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv,
+                                     int64_t kv_stride_0, int64_t kv_stride_1, int64_t num_blocks,
+                                     int32_t page_size, const int32_t* block_table, int64_t bt_stride_b,
+                                     int32_t bt_cols, const int32_t* seqlens, int32_t batch, int32_t num_heads,
+                                     int32_t head_dim_v, int32_t rope_dim, int32_t dtype, float softmax_scale,
+                                     int32_t num_workers, void* out, int64_t out_stride_b, int64_t out_stride_h,
+                                     float* lse, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Profiling hook, no counterpart in the reference: copies the partial

@@ -152,6 +152,33 @@ def test_generic_workspace_and_rejections(lib):
     assert lib.tmla_generic_heads_per_workgroup(128, 32, 2) == 16
     assert lib.tmla_generic_heads_per_workgroup(96, 32, 0) == 0
     assert lib.tmla_generic_heads_per_workgroup(128, 32, 3) == 0
+
+
+def test_generic_balanced_workers_and_rejections(lib):
+    """The balanced generic call: its worker counts (one resident workgroup
+    per compute unit; two in float32 up to 256 dims; shared along the heads),
+    its workspace and what it refuses."""
+    w = lib.tmla_generic_workers
+    assert w(256, 32, 0, 128, 256) == 256 and w(256, 32, 0, 129, 256) == 128 and w(512, 16, 1, 300, 256) == 85
+    assert w(512, 64, 2, 16, 256) == 256 and w(256, 64, 2, 16, 256) == 512 and w(512, 64, 2, 33, 256) == 128
+    assert w(64, 16, 0, 65535, 256) == 1
+    for dv, dr, dt, heads in ((32, 16, 0, 8), (1024, 64, 0, 8), (256, 128, 0, 8), (256, 32, 3, 8), (256, 32, 0, 0)):
+        assert w(dv, dr, dt, heads, 256) == 0
+    need = lib.tmla_generic_balanced_workspace_bytes
+    assert need(2, 16, 128, 256) == lib.tmla_generic_workspace_bytes(258, 16, 128, 1)
+    assert need(2, 16, 128, 0) == 0 and need(2**31 - 1, 16, 128, 1) == 0
+    fake = 1 << 20
+
+    def call(dv=256, dr=32, workers=256, wsb=None, q=fake, stride=288, batch=2):
+        return lib.tmla_mla_decode_generic_balanced(
+            q, 16 * stride, stride, fake, 64 * stride, stride, 8, 64, fake, 4, 4, fake, batch, 16, dv, dr, 0, 0.1,
+            workers, fake, 16 * dv, dv, None, fake, need(2, 16, dv, 256) if wsb is None else wsb, None)
+
+    assert call(workers=0) == 1 and call(workers=65536, wsb=1 << 50) == 1
+    assert call(wsb=need(2, 16, 256, 256) - 1) == 3
+    assert call(dv=32, dr=16) == 2 and call(dr=128) == 2  # dims the kernels do not take
+    assert call(q=fake + 2) == 2 and call(stride=289) == 2  # rows off 16-byte boundaries
+    assert call(q=None) == 1 and call(batch=0) == 0
     # the matrix-core entry points keep refusing float32
     assert _partial(lib, dtype=2, ws=fake, wsb=lib.tmla_workspace_bytes(2, 128, 512, 1, 0)) == 1
 

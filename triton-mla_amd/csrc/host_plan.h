@@ -257,6 +257,27 @@ inline int generic_mfma_form(int32_t dv, int32_t dr, int32_t dtype) {
   return need <= kGenMfmaSmallLds ? kGenMfmaSmallLds : (need <= kGenMfmaLargeLds ? kGenMfmaLargeLds : 0);
 }
 
+// The matrix-core kernels of other dims and float32 (mla_decode_dims.hip):
+// rows whose latent part is whole 128-byte blocks and whose rope part is at
+// most one, read in 16-byte pieces.
+inline bool dims_form(int32_t dv, int32_t dr) {
+  return (dv == 64 || dv == 128 || dv == 256 || dv == 512) && (dr == 16 || dr == 32 || dr == 64);
+}
+// Heads per workgroup: 128 (32 per wave) in 16 bits; 16 or 32 in float32.
+inline int32_t dims_heads_per_workgroup(int32_t dtype, int32_t heads) {
+  return dtype != TMLA_FP32 ? 128 : heads <= 16 ? 16 : 32;
+}
+// Workers of the balanced partition: the workgroups that are resident at
+// once (one per compute unit by their LDS; two in float32 up to 256 value
+// dims), shared by the workgroups along the heads.
+inline int32_t dims_workers(int32_t dv, int32_t dtype, int32_t heads, int32_t cus) {
+  const int64_t per = dims_heads_per_workgroup(dtype, heads);
+  const int64_t gy = ((int64_t)heads + per - 1) / per;
+  const int64_t resident = (int64_t)cus * (dtype == TMLA_FP32 && dv <= 256 ? 2 : 1);
+  return (int32_t)(resident / gy > 0 ? resident / gy : 1);
+}
+constexpr int64_t kDimsMaxGrid = 1 << 22;  // workgroups along x (512 threads each)
+
 // Workspace of a generic call: the float32 partial rows, then their lse
 // values (both 256-byte aligned); 0 for invalid or too large arguments.
 inline size_t generic_workspace_bytes(int32_t batch, int32_t heads, int32_t dv, int32_t splits) {
@@ -268,6 +289,12 @@ inline size_t generic_workspace_bytes(int32_t batch, int32_t heads, int32_t dv, 
   auto al = [](int64_t x) { return (x + 255) & ~(int64_t)255; };
   const int64_t total = al(rows * dv * 4) + al(rows * 4) + 256;
   return total > kMaxWorkspaceBytes ? 0 : (size_t)total;
+}
+
+// Workspace of a balanced generic call: num_workers + batch slots.
+inline size_t generic_balanced_workspace_bytes(int32_t batch, int32_t heads, int32_t dv, int32_t workers) {
+  if (batch < 0 || workers <= 0 || batch > INT32_MAX - workers) return 0;
+  return generic_workspace_bytes(batch + workers, heads, dv, 1);
 }
 
 struct GenericCall {

@@ -41,6 +41,7 @@
 #include <stdio.h>
 
 #include "cdna.h"
+#include "dims.h"
 #include "host_plan.h"
 #include "triton_mla.h"
 
@@ -684,31 +685,33 @@ extern int hip_fail(hipError_t e, const char* where);
 
 }  // namespace tmla
 
-using namespace tmla;
+namespace tmla {
 
-extern "C" {
-
-size_t tmla_generic_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim_v, int32_t num_splits) {
-  return generic_workspace_bytes(batch, num_heads, head_dim_v, num_splits);
-}
-
-int32_t tmla_generic_heads_per_workgroup(int32_t head_dim_v, int32_t rope_dim, int32_t dtype) {
-  if (dtype != TMLA_BF16 && dtype != TMLA_FP16 && dtype != TMLA_FP32) return 0;
-  if (!pow2_between(head_dim_v, 16, 1024) || !pow2_between(rope_dim, 16, 256)) return 0;
-  return generic_mfma_form(head_dim_v, rope_dim, dtype) != 0 ? kGenMfmaHeads : kGenHeads;
-}
-
-int tmla_mla_decode_generic(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv,
-                            int64_t kv_stride_0, int64_t kv_stride_1, int64_t num_blocks, int32_t page_size,
-                            const int32_t* block_table, int64_t bt_stride_b, int32_t bt_cols,
-                            const int32_t* seqlens, int32_t batch, int32_t num_heads, int32_t head_dim_v,
-                            int32_t rope_dim, int32_t dtype, float softmax_scale, int32_t num_splits, void* out,
-                            int64_t out_stride_b, int64_t out_stride_h, float* lse, void* workspace,
-                            size_t workspace_bytes_, void* stream) {
+// Both entry points: num_splits >= 1 cuts every sequence into that many
+// pieces; num_splits == 0 (tmla_mla_decode_generic_balanced) spreads the
+// tiles of all sequences over num_workers ranges, in mla_decode_dims.hip only.
+static int generic_call(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv, int64_t kv_stride_0,
+                        int64_t kv_stride_1, int64_t num_blocks, int32_t page_size, const int32_t* block_table,
+                        int64_t bt_stride_b, int32_t bt_cols, const int32_t* seqlens, int32_t batch,
+                        int32_t num_heads, int32_t head_dim_v, int32_t rope_dim, int32_t dtype, float softmax_scale,
+                        int32_t num_splits, int32_t num_workers, void* out, int64_t out_stride_b,
+                        int64_t out_stride_h, float* lse, void* workspace, size_t workspace_bytes_, void* stream) {
   const bool paged = block_table != nullptr;
-  const GenericCall c{batch, num_heads, head_dim_v, rope_dim, dtype, num_splits,
+  const bool balanced = num_splits == 0;
+  // (the balanced form's slots: one per worker and one more per sequence)
+  const GenericCall c{batch, num_heads, head_dim_v, rope_dim, dtype, balanced ? 1 : num_splits,
                       paged, page_size, bt_cols, num_blocks};
-  const int rc = check_generic(c, workspace, workspace_bytes_);
+  int rc;
+  if (balanced) {
+    if (num_workers <= 0 || num_workers > kGenMaxBatchHeads)
+      return fail(TMLA_ERR_INVALID_ARGUMENT, "num_workers must be in [1, 65535]");
+    const size_t need = generic_balanced_workspace_bytes(batch, num_heads, head_dim_v, num_workers);
+    rc = check_generic(c, workspace, workspace_bytes_);
+    if (rc == TMLA_OK && (need == 0 || workspace_bytes_ < need))
+      rc = fail(TMLA_ERR_WORKSPACE_TOO_SMALL, "workspace is smaller than tmla_generic_balanced_workspace_bytes()");
+  } else {
+    rc = check_generic(c, workspace, workspace_bytes_);
+  }
   if (rc != TMLA_OK) return rc;
   if (batch == 0) return TMLA_OK;
   if (q == nullptr || kv == nullptr || seqlens == nullptr || out == nullptr)
@@ -740,7 +743,7 @@ int tmla_mla_decode_generic(const void* q, int64_t q_stride_b, int64_t q_stride_
   a.pitch = p.pitch;
   a.vec = ((uintptr_t)kv % 16 == 0 && (kv_stride_0 * es) % 16 == 0 && (kv_stride_1 * es) % 16 == 0) ? 1 : 0;
   a.qvec = ((uintptr_t)q % 16 == 0 && (q_stride_b * es) % 16 == 0 && (q_stride_h * es) % 16 == 0) ? 1 : 0;
-  const int64_t rows = (int64_t)batch * num_heads * num_splits;
+  const int64_t rows = (int64_t)num_heads * (balanced ? (int64_t)num_workers + batch : (int64_t)batch * num_splits);
   a.mid_o = (float*)workspace;
   a.mid_lse = (float*)((char*)workspace + ((rows * head_dim_v * 4 + 255) & ~(int64_t)255));
   a.out = (char*)out;
@@ -748,12 +751,110 @@ int tmla_mla_decode_generic(const void* q, int64_t q_stride_b, int64_t q_stride_
   a.out_sh = out_stride_h;
   a.lse = lse;
   hipStream_t st = (hipStream_t)stream;
+  // the matrix-core kernels of the usual dims: rows and output in 16-byte pieces
+  const bool ovec = (uintptr_t)out % 16 == 0 && (out_stride_b * es) % 16 == 0 && (out_stride_h * es) % 16 == 0;
+  // (a float32 call of a given split count keeps the vector-ALU form, whose
+  // bits do not depend on the rows' alignment)
+  const bool dims_fit =
+      dims_form(head_dim_v, rope_dim) && a.vec && a.qvec && ovec &&
+      (balanced || (dtype != TMLA_FP32 && (int64_t)batch * num_splits <= kDimsMaxGrid));
+  if (balanced && !dims_fit)
+    return fail(TMLA_ERR_UNSUPPORTED, "the balanced generic decode needs head_dim_v 64 to 512, rope_dim 16 to 64 and "
+                                      "16-byte aligned q, kv and out rows");
+  if (dims_fit) {
+    dims::DimsArgs d{};
+    d.q = a.q;
+    d.q_sb = q_stride_b;
+    d.q_sh = q_stride_h;
+    d.kv = a.kv;
+    d.kv_s0 = kv_stride_0 * es;
+    d.kv_s1 = kv_stride_1 * es;
+    d.num_blocks = num_blocks;
+    d.max_page = (int32_t)(num_blocks - 1 < INT32_MAX ? num_blocks - 1 : INT32_MAX);
+    d.page_size = page_size;
+    d.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz((unsigned)page_size) : -1;
+    d.bt = block_table;
+    d.bt_sb = bt_stride_b;
+    d.bt_cols = bt_cols;
+    d.seqlens = seqlens;
+    d.batch = batch;
+    d.num_heads = num_heads;
+    d.q_len = 1;
+    d.heads_per_token = num_heads;
+    // (a zero scale would make masked scores NaN: the smallest normal instead)
+    d.qk_scale_log2 = a.qk_scale == 0.0f && dtype != TMLA_FP32 ? 1.17549435e-38f : a.qk_scale;
+    d.num_splits = num_splits;
+    d.num_workers = num_workers;
+    d.xcds = 8;
+    d.out = a.out;
+    d.out_sb = out_stride_b;
+    d.out_sh = out_stride_h;
+    d.lse = lse;
+    d.len_cap = (int32_t)(a.capacity < INT32_MAX - 128 ? a.capacity : INT32_MAX - 128);
+    d.uni = (!paged || page_size % (dtype == TMLA_FP32 ? 16 : 32) == 0) && d.kv_s1 > 0 && d.kv_s1 < (1 << 26) ? 1 : 0;
+    d.part = a.mid_o;
+    d.part_lse = a.mid_lse;
+    const hipError_t e = dims::launch(d, head_dim_v, rope_dim, dtype, a.capacity, (hipStream_t)stream);
+    return e == hipSuccess ? TMLA_OK : hip_fail(e, "mla_dims kernels launch");
+  }
   // the matrix-core form reads q and the cache in 16-byte pieces only
   const int mfma_lds = a.vec && a.qvec ? generic_mfma_form(head_dim_v, rope_dim, dtype) : 0;
   const hipError_t e = dtype == TMLA_BF16   ? gen::launch_t<TMLA_BF16>(a, p.lds, mfma_lds, st)
                        : dtype == TMLA_FP16 ? gen::launch_t<TMLA_FP16>(a, p.lds, mfma_lds, st)
                                             : gen::launch_t<TMLA_FP32>(a, p.lds, mfma_lds, st);
   return e == hipSuccess ? TMLA_OK : hip_fail(e, "mla_generic kernels launch");
+}
+
+}  // namespace tmla
+
+using namespace tmla;
+
+extern "C" {
+
+size_t tmla_generic_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim_v, int32_t num_splits) {
+  return generic_workspace_bytes(batch, num_heads, head_dim_v, num_splits);
+}
+
+int32_t tmla_generic_heads_per_workgroup(int32_t head_dim_v, int32_t rope_dim, int32_t dtype) {
+  if (dtype != TMLA_BF16 && dtype != TMLA_FP16 && dtype != TMLA_FP32) return 0;
+  if (!pow2_between(head_dim_v, 16, 1024) || !pow2_between(rope_dim, 16, 256)) return 0;
+  return generic_mfma_form(head_dim_v, rope_dim, dtype) != 0 ? kGenMfmaHeads : kGenHeads;
+}
+
+int tmla_mla_decode_generic(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv,
+                            int64_t kv_stride_0, int64_t kv_stride_1, int64_t num_blocks, int32_t page_size,
+                            const int32_t* block_table, int64_t bt_stride_b, int32_t bt_cols,
+                            const int32_t* seqlens, int32_t batch, int32_t num_heads, int32_t head_dim_v,
+                            int32_t rope_dim, int32_t dtype, float softmax_scale, int32_t num_splits, void* out,
+                            int64_t out_stride_b, int64_t out_stride_h, float* lse, void* workspace,
+                            size_t workspace_bytes_, void* stream) {
+  if (num_splits < 1) num_splits = -1;  // refused (0 is the balanced form's)
+  return generic_call(q, q_stride_b, q_stride_h, kv, kv_stride_0, kv_stride_1, num_blocks, page_size, block_table,
+                      bt_stride_b, bt_cols, seqlens, batch, num_heads, head_dim_v, rope_dim, dtype, softmax_scale,
+                      num_splits, 0, out, out_stride_b, out_stride_h, lse, workspace, workspace_bytes_, stream);
+}
+
+int32_t tmla_generic_workers(int32_t head_dim_v, int32_t rope_dim, int32_t dtype, int32_t num_heads, int32_t cus) {
+  if (dtype != TMLA_BF16 && dtype != TMLA_FP16 && dtype != TMLA_FP32) return 0;
+  if (num_heads <= 0 || cus <= 0 || !dims_form(head_dim_v, rope_dim)) return 0;
+  return dims_workers(head_dim_v, dtype, num_heads, cus);
+}
+
+size_t tmla_generic_balanced_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim_v,
+                                             int32_t num_workers) {
+  return generic_balanced_workspace_bytes(batch, num_heads, head_dim_v, num_workers);
+}
+
+int tmla_mla_decode_generic_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv,
+                                     int64_t kv_stride_0, int64_t kv_stride_1, int64_t num_blocks,
+                                     int32_t page_size, const int32_t* block_table, int64_t bt_stride_b,
+                                     int32_t bt_cols, const int32_t* seqlens, int32_t batch, int32_t num_heads,
+                                     int32_t head_dim_v, int32_t rope_dim, int32_t dtype, float softmax_scale,
+                                     int32_t num_workers, void* out, int64_t out_stride_b, int64_t out_stride_h,
+                                     float* lse, void* workspace, size_t workspace_bytes_, void* stream) {
+  return generic_call(q, q_stride_b, q_stride_h, kv, kv_stride_0, kv_stride_1, num_blocks, page_size, block_table,
+                      bt_stride_b, bt_cols, seqlens, batch, num_heads, head_dim_v, rope_dim, dtype, softmax_scale, 0,
+                      num_workers, out, out_stride_b, out_stride_h, lse, workspace, workspace_bytes_, stream);
 }
 
 }  // extern "C"

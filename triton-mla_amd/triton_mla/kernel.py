@@ -458,12 +458,12 @@ def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax
     are not built for (tmla_mla_decode_generic): any power-of-two head_dim_v
     in [16, 1024] and rope_dim in [16, 256], bf16, fp16 or fp32 -- the
     reference's kernels take powers of two and any dtype q and the cache
-    share (kernel.py:243-245). Both of the reference's stages with its
-    uniform splits (kernel.py:84-86) and float32 partials; ``num_splits=None``
-    takes _generic_splits of the cache's capacity (sized for the form's
-    workgroups: 64 heads on matrix cores for bf16 / fp16 up to 512 + 64, 16
-    on the vector ALU otherwise; no call reads ``cache_seqlens`` back to the
-    host). Meant for unusual dims, not at the 512 + 64 kernels' speed."""
+    share (kernel.py:243-245). Both of the reference's stages with float32
+    partials. ``num_splits=None`` runs the balanced partition
+    (tmla_mla_decode_generic_balanced) at head_dim_v 64 to 512, rope_dim 16 to
+    64 and 16-byte aligned rows; elsewhere it takes _generic_splits uniform
+    pieces (kernel.py:84-86) of the cache's capacity. No call reads
+    ``cache_seqlens`` back to the host."""
     # validation mirrors kernel.py:235-245
     if kv_cache.dim() == 4:
         assert kv_cache.shape[2] == 1, "MLA uses a single shared latent KV head"
@@ -504,27 +504,41 @@ def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax
         page_size, num_blocks = 1, kv_cache.shape[1]
         capacity = num_blocks
         bt_args = (None, 0, 1)
+    lib = _native.load()
+    dtype = _native.DTYPE_CODE[q.dtype]
+    workers = 0
     if num_splits is None:
-        per_wg = _native.load().tmla_generic_heads_per_workgroup(head_dim_v, d_rope, _native.DTYPE_CODE[q.dtype])
-        num_splits = _generic_splits(batch, num_heads, capacity, _num_sms(device), max(per_wg, 1))
-    num_splits = int(num_splits)
-    assert num_splits >= 1, "num_splits must be >= 1"
+        # the balanced partition where its kernels take the call (the usual
+        # dims, rows on 16-byte boundaries), uniform pieces otherwise
+        elems = 16 // q.element_size()
+        if _aligned(q, elems) and _aligned(kv_cache, elems):
+            workers = lib.tmla_generic_workers(head_dim_v, d_rope, dtype, num_heads, _num_sms(device))
+        if workers == 0:
+            per_wg = lib.tmla_generic_heads_per_workgroup(head_dim_v, d_rope, dtype)
+            num_splits = _generic_splits(batch, num_heads, capacity, _num_sms(device), max(per_wg, 1))
+    if workers == 0:
+        num_splits = int(num_splits)
+        assert num_splits >= 1, "num_splits must be >= 1"
     out = torch.empty(batch, num_heads, head_dim_v, dtype=q.dtype, device=device)
     lse = torch.empty(batch, num_heads, dtype=torch.float32, device=device)
     if batch:
         if block_table is not None and num_blocks == 0:
             raise ValueError("kv_cache holds no pages")
-        lib = _native.load()
-        ws_bytes = lib.tmla_generic_workspace_bytes(batch, num_heads, head_dim_v, num_splits)
+        if workers:
+            fn, parts = lib.tmla_mla_decode_generic_balanced, workers
+            ws_bytes = lib.tmla_generic_balanced_workspace_bytes(batch, num_heads, head_dim_v, workers)
+        else:
+            fn, parts = lib.tmla_mla_decode_generic, num_splits
+            ws_bytes = lib.tmla_generic_workspace_bytes(batch, num_heads, head_dim_v, num_splits)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
         dev_idx = device.index if device.index is not None else torch.cuda.current_device()
         with _OnDevice(dev_idx):
-            _native.check(lib.tmla_mla_decode_generic(
+            _native.check(fn(
                 q.data_ptr(), q.stride(0), q.stride(1), kv_cache.data_ptr(), kv_cache.stride(0), kv_cache.stride(1),
                 num_blocks, page_size, *bt_args, cache_seqlens.data_ptr(), batch, num_heads, head_dim_v, d_rope,
-                _native.DTYPE_CODE[q.dtype], float(softmax_scale), num_splits, out.data_ptr(), out.stride(0),
-                out.stride(1), lse.data_ptr(), workspace.data_ptr(), ws_bytes,
-                torch.cuda.current_stream(device).cuda_stream), "tmla_mla_decode_generic")
+                dtype, float(softmax_scale), parts, out.data_ptr(), out.stride(0), out.stride(1), lse.data_ptr(),
+                workspace.data_ptr(), ws_bytes, torch.cuda.current_stream(device).cuda_stream),
+                "tmla_mla_decode_generic")
     if return_lse:
         return out, lse
     return out
