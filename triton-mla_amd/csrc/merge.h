@@ -77,7 +77,7 @@ __device__ __forceinline__ void merge_zero(const MergeView& mv, int b, int head,
   if (lane == 0 && mv.lse) mv.lse[(int64_t)b * mv.num_heads + head] = -INFINITY;
 }
 
-// Heads [head, head + nh), nh <= NH, over slots [slot0, slot0 + count),
+// The single launch's merge of heads [head, head + nh), nh <= NH, over slots [slot0, slot0 + count),
 // count <= NR: every lse and row load is issued before the first use. Slots
 // past `count` repeat the last one with weight 0; heads past `nh` repeat the
 // last head and are not stored.
@@ -146,6 +146,107 @@ __device__ __forceinline__ void merge_row_loop(const MergeView& mv, const LD& ld
       wsum += w[j];
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[e] += w[j] * Elt<DT>::to_float(v[j][e]);
+    }
+  }
+  merge_store<DT>(mv, b, head, acc, wsum, m, lane);
+}
+
+// Max over aligned groups of G lanes (8, 16, 32 or 64), by DPP moves and row
+// swaps (no LDS round trips).
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float x) {
+  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true)));
+}
+template <int G>
+__device__ __forceinline__ float group_max(float x) {
+  x = dpp_max<0xB1>(x);                            // lane ^ 1
+  x = dpp_max<0x4E>(x);                            // lane ^ 2
+  x = dpp_max<0x141>(x);                           // the other half of 8
+  if constexpr (G >= 16) x = dpp_max<0x140>(x);    // the other half of 16
+  if constexpr (G >= 32) {
+    float y = x;
+    swap_rows16(x, y);
+    x = fmaxf(x, y);
+  }
+  if constexpr (G >= 64) {
+    float y = x;
+    swap_rows32(x, y);
+    x = fmaxf(x, y);
+  }
+  return x;
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+
+// The combine kernel's merge (stage 2) of heads [head, head + nh), nh <= NH,
+// over slots [slot0, slot0 + count), count <= NR: the results of
+// merge_rows_at_once bit for bit (the same max, weights and order of sums).
+// One load gives lane i * NR + j the lse of head i's slot j, and with it the wave computes every
+// weight once; the row loads are issued beside it, before the first use. Slots
+// past `count` repeat the last one with weight 0; heads past `nh` repeat the
+// last head and are not stored.
+template <int DT, int NH, int NR, class LD>
+__device__ __forceinline__ void combine_rows(const MergeView& mv, const LD& ld, int b, int head, int nh,
+                                                   int slot0, int count, int lane) {
+  static_assert(NH * NR <= 64, "one lse per lane");
+  i16x8 v[NH][NR];
+  // row indices in VGPRs: vector address arithmetic instead of one scalar
+  // register pair per row
+  int r0 = slot0 * mv.num_heads + head;
+  pin_i1(r0);
+  const int li = lane / NR, lj = lane % NR;
+  const float lv = ld.lse((int64_t)(r0 + min(lj, count - 1) * mv.num_heads + min(li, nh - 1)));
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    const int hh = min(i, nh - 1);
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      v[i][j] = ld.rowv((int64_t)(r0 + min(j, count - 1) * mv.num_heads + hh), lane);
+  }
+  const float l = lj < count ? lv : -INFINITY;
+  float m = group_max<NR>(l);
+  if (m == -INFINITY) m = 0.0f;
+  const float w = lj < count ? fast_exp2(l - m) : 0.0f;
+#pragma unroll
+  for (int i = 0; i < NH; ++i) {
+    if (i >= nh) break;
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, wsum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      const float wj = lane_value(w, i * NR + j);
+      wsum += wj;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += wj * Elt<DT>::to_float(v[i][j][e]);
+    }
+    merge_store<DT>(mv, b, head + i, acc, wsum, lane_value(m, i * NR), lane);
+  }
+}
+
+// Any count: the max over all slots first, then NR rows in flight per batch.
+// The result does not depend on NR, and equals combine_rows over the
+// same slots bit for bit (the same max, weights and order of sums).
+template <int DT, int NR, class LD>
+__device__ __forceinline__ void combine_row_loop(const MergeView& mv, const LD& ld, int b, int head, int slot0,
+                                               int count, int lane) {
+  float m = -INFINITY;
+  for (int s = lane; s < count; s += 64) m = fmaxf(m, ld.lse((int64_t)(slot0 + s) * mv.num_heads + head));
+  m = group_max<64>(m);
+  if (m == -INFINITY) m = 0.0f;
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, wsum = 0.0f;
+  for (int s0 = 0; s0 < count; s0 += NR) {
+    i16x8 v[NR];
+    const float lv = ld.lse((int64_t)(slot0 + min(s0 + lane % NR, count - 1)) * mv.num_heads + head);
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      v[j] = ld.rowv((int64_t)(slot0 + min(s0 + j, count - 1)) * mv.num_heads + head, lane);
+    const float w = s0 + lane % NR < count ? fast_exp2(lv - m) : 0.0f;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+      const float wj = lane_value(w, j);
+      wsum += wj;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += wj * Elt<DT>::to_float(v[j][e]);
     }
   }
   merge_store<DT>(mv, b, head, acc, wsum, m, lane);

@@ -1108,7 +1108,7 @@ void mla_partial_kernel(PartialArgs a) {
       // the page-id (and scale) loads go out before every counted LDS read of
       // the iteration, so their out-of-order returns can only make the
       // counted waits wait longer
-      if (PAGED && PAGE_UNIFORM && i + kStages < nst)
+      if (PAGED && PAGE_UNIFORM && do_copy && i + kStages < nst)
         next_page = i < 0 ? pro_page[kStages - 1] : page_fetch(st0 + i + kStages);
       if (F8 && do_copy) sc3 = s_load_f32(a.kv_scale + (int64_t)page * a.sc_s0);  // sub-tile i+3
       const int pbuf = i & 1;
@@ -2130,37 +2130,41 @@ void mla_partial_own_kernel(PartialArgs a) {
 // heads of sequence b: one head per wave (HPW = 1), or, for calls with many
 // (sequence, head) pairs, four heads per wave (HPW = 4) so that every
 // workgroup fits the compute units in one round and each wave has four
-// heads' rows in flight. Both give the same bits.
+// heads' rows in flight. Both give the same bits. What bounds it is the chain
+// lengths -> slots -> partial rows, each a memory round trip, so a wave
+// issues every load of its rows at once, and one load for all their lse
+// values (a load and an exponential per slot and lane before: 4 sequences of
+// 32K tokens, 64 partials a row, 75.5 us per call instead of 59). Sharing a
+// row among four waves where rows are few was measured too: no difference.
 // ---------------------------------------------------------------------------
 template <int DT, int DV, int HPW>
 __global__ __launch_bounds__(256) void mla_combine_kernel(CombineArgs a) {
-  static_assert(DV % 256 == 0, "8 dims per lane");
+  static_assert(DV == 512, "one row = 64 lanes x 8 elements");
   static_assert(HPW == 1 || HPW == 4, "one or four heads per wave");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = blockIdx.x;
-  const int h_lo = blockIdx.y * 4 * HPW;
-  const int h_hi = min(h_lo + 4 * HPW, a.num_heads);
-
   int slot0, count;
   sequence_slots(GivenLens{a.seqlens}, a.batch, a.num_splits, a.num_workers, b, slot0, count);
   if (count == 1) return;  // written by stage 1
-  static_assert(DV == 512, "one row = 64 lanes x 8 elements");
   const MergeView mv{a.mid_o, a.mid_lse, a.num_heads, a.out, a.out_sb, a.out_sh, a.lse};
   const PlainLoads ld{a.mid_o, a.mid_lse};
+  const int h_lo = blockIdx.y * 4 * HPW;
+  const int h_hi = min(h_lo + 4 * HPW, a.num_heads);
   if (count == 0) {
     for (int h = h_lo + wave; h < h_hi; h += 4) merge_zero(mv, b, h, lane);
   } else if (count <= 8) {
     // HPW heads of one wave together: HPW * count rows in flight
     const int h = h_lo + HPW * wave;
-    if (h < h_hi) merge_rows_at_once<DT, HPW, 8>(mv, ld, b, h, min(HPW, h_hi - h), slot0, count, lane);
+    if (h < h_hi) combine_rows<DT, HPW, 8>(mv, ld, b, h, min(HPW, h_hi - h), slot0, count, lane);
   } else if (count <= 16) {
     constexpr int P = HPW == 4 ? 2 : 1;  // heads per pass
     for (int h = h_lo + P * wave; h < h_hi; h += 4 * P)
-      merge_rows_at_once<DT, P, 16>(mv, ld, b, h, min(P, h_hi - h), slot0, count, lane);
+      combine_rows<DT, P, 16>(mv, ld, b, h, min(P, h_hi - h), slot0, count, lane);
   } else if (count <= 32) {  // e.g. a few long sequences cut over all workers: one round trip
-    for (int h = h_lo + wave; h < h_hi; h += 4) merge_rows_at_once<DT, 1, 32>(mv, ld, b, h, 1, slot0, count, lane);
+    for (int h = h_lo + wave; h < h_hi; h += 4)
+      combine_rows<DT, 1, 32>(mv, ld, b, h, 1, slot0, count, lane);
   } else {
-    for (int h = h_lo + wave; h < h_hi; h += 4) merge_row_loop<DT, 32>(mv, ld, b, h, slot0, count, lane);
+    for (int h = h_lo + wave; h < h_hi; h += 4) combine_row_loop<DT, 32>(mv, ld, b, h, slot0, count, lane);
   }
 }
 
@@ -2201,6 +2205,15 @@ struct Fp8Scales {
   const float* scale;
   int64_t s0, s1;
 };
+
+template <int HPW>
+hipError_t launch_combine_t(const CombineArgs& a, int dtype, dim3 grid, hipStream_t stream) {
+  if (dtype == TMLA_BF16)
+    hipLaunchKernelGGL((mla_combine_kernel<TMLA_BF16, 512, HPW>), grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((mla_combine_kernel<TMLA_FP16, 512, HPW>), grid, dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
 
 template <int DT, int NHB, bool PAGED, bool UNI, bool F8 = false>
 hipError_t launch_partial_t(const PartialArgs& a, dim3 grid, hipStream_t stream) {
@@ -2503,20 +2516,9 @@ int tmla_mla_decode_combine(const int32_t* seqlens, int32_t batch, int32_t num_h
   hipStream_t s = static_cast<hipStream_t>(stream);
   // four heads per wave once one head per wave would take more than
   // kCombineWideWgs workgroups
-  const bool wide = (int64_t)batch * ((num_heads + 3) / 4) > kCombineWideWgs;
-  const dim3 grid(batch, wide ? (num_heads + 15) / 16 : (num_heads + 3) / 4);
-  if (dtype == TMLA_BF16) {
-    if (wide)
-      hipLaunchKernelGGL((mla_combine_kernel<TMLA_BF16, 512, 4>), grid, dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((mla_combine_kernel<TMLA_BF16, 512, 1>), grid, dim3(256), 0, s, a);
-  } else {
-    if (wide)
-      hipLaunchKernelGGL((mla_combine_kernel<TMLA_FP16, 512, 4>), grid, dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((mla_combine_kernel<TMLA_FP16, 512, 1>), grid, dim3(256), 0, s, a);
-  }
-  hipError_t e = hipGetLastError();
+  const hipError_t e = (int64_t)batch * ((num_heads + 3) / 4) > kCombineWideWgs
+                           ? launch_combine_t<4>(a, dtype, dim3(batch, (num_heads + 15) / 16), s)
+                           : launch_combine_t<1>(a, dtype, dim3(batch, (num_heads + 3) / 4), s);
   if (e != hipSuccess) return hip_fail(e, "mla_combine_kernel launch");
   return TMLA_OK;
 }
