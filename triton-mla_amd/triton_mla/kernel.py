@@ -106,6 +106,21 @@ def balanced_pieces(seqlens, num_workers: int, segment_tiles: int = SEGMENT_STAR
     return best
 
 
+def _balanced_workers(num_sms: int, heads: int, heads_per_workgroup: int, tiles: int) -> int:
+    """Workers of the balanced partition: the compute units, shared by the
+    workgroups a worker's range takes along the (virtual) heads, since each
+    round of workgroups pays its start-up, its finalize and its partials
+    again (16 sequences of 1K to 8K tokens, two query tokens of 128 heads:
+    79 us with 256 workers in two rounds, 59 us with 128 in one).
+    Calls whose cache holds fewer than four 64-token tiles per compute unit
+    keep one worker per compute unit, the partition (and so the bits) of a
+    single-token call."""
+    groups = _cdiv(heads, heads_per_workgroup)
+    if groups == 1 or tiles < 4 * num_sms:
+        return num_sms
+    return max(1, num_sms // groups)
+
+
 # The form mla_decode runs when single_launch is None: False = the two
 # kernels of the reference's scheme (partial, then combine), True = the single
 # launch (the merge inside the partial kernel, same bits) whenever its
@@ -263,8 +278,19 @@ class DecodeLaunch:
         self._keep = (q, kv_cache, cache_seqlens, block_table, kv_scale)
         self.lib = _native.load()
         self.splits = num_splits if num_splits is not None else 0
+        capacity = (block_table.shape[1] * page_size) if block_table is not None else num_blocks
         # balanced partition: one worker per compute unit unless asked otherwise
-        self.workers = 0 if num_splits is not None else int(num_workers or _num_sms(device))
+        self.workers = 0
+        if num_splits is None:
+            if num_workers:
+                self.workers = int(num_workers)
+            else:
+                # heads per workgroup: 128, or 16 for an fp8 cache whose pages
+                # are not widened into the 16-bit ring
+                ring = not fp8 or (scale_args[2] == 0 and block_table is not None and page_size % 32 == 0
+                                   and page_size & (page_size - 1) == 0)
+                self.workers = _balanced_workers(_num_sms(device), vheads, 128 if ring else 16,
+                                                 batch * _cdiv(capacity, 64))
         dev_idx = device.index if device.index is not None else torch.cuda.current_device()
         self._dev_idx = dev_idx
         # The library's answers for this shape (workspace size, the counter
@@ -272,7 +298,6 @@ class DecodeLaunch:
         # launch) depend on the shape and device only: asked once per shape.
         # run(single_launch=True) merges inside the partial kernel when all of
         # its workgroups fit on the device at once, one per CU.
-        capacity = (block_table.shape[1] * page_size) if block_table is not None else num_blocks
         key = (dev_idx, batch, vheads, head_dim_v, self.splits, self.workers, capacity, fp8, id(self.lib))
         plan = _PLANS.get(key)
         if plan is None:
