@@ -116,3 +116,55 @@ def test_graph_capture_and_threads_share_no_workspace():
     for i, outs in results.items():
         ref = ref_a if i % 2 == 0 else ref_b
         assert all(torch.equal(o, ref) for o in outs), f"thread {i}"
+
+
+@pytest.mark.parametrize("kind", ["fp8_page", "fp8_token", "fp8_two_tokens", "two_tokens", "dims", "fp32"])
+def test_repeated_other_shapes_match_a_fresh_launch(kind):
+    """fp8, multi-token and generic calls of a shape seen before (their
+    arguments' addresses in the kept ones, the stream's workspace) give the
+    bits of a first call, with new contents and buffers each time, on a
+    second stream and captured in a graph."""
+    dev = torch.device("cuda:0")
+
+    def call(seed):
+        q, kv, seqlens, bt = _inputs(seed)
+        kw = dict(softmax_scale=SCALE, return_lse=True)
+        if kind == "dims":
+            q, kv, kw["head_dim_v"] = q[..., :288].contiguous(), kv[..., :288].contiguous(), 256
+        elif kind == "fp32":
+            q, kv = q.float(), kv.float()
+        if kind in ("two_tokens", "fp8_two_tokens"):
+            q = torch.stack([q, -q], dim=1).contiguous()
+        q, kv, seqlens, bt = (t.to(dev) for t in (q, kv, seqlens, bt))
+        if kind.startswith("fp8"):
+            kv, kw["kv_scale"] = triton_mla.quantize_kv_fp8(kv, "token" if kind == "fp8_token" else "page")
+        return (q, kv, seqlens, bt), kw
+
+    K._OTHER_SHAPES.clear()
+    fresh, again = [], []
+    for seed in range(3):
+        args, kw = call(seed)
+        K._OTHER_SHAPES.clear()
+        fresh.append(triton_mla.mla_decode(*args, **kw))
+    for seed in range(3):
+        args, kw = call(seed)
+        again.append(triton_mla.mla_decode(*args, **kw))
+    assert any(K._OTHER_SHAPES.values()), "the repeated shape did not take the kept-argument path"
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        other = triton_mla.mla_decode(*args, **kw)
+    torch.cuda.synchronize()
+    for f, a in zip(fresh, again):
+        assert torch.equal(f[0], a[0]) and torch.equal(f[1], a[1])
+    assert torch.equal(other[0], fresh[2][0]) and torch.equal(other[1], fresh[2][1])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        g_out, g_lse = triton_mla.mla_decode(*args, **kw)
+    for _ in range(3):
+        g_out.zero_()
+        with torch.cuda.stream(side):
+            graph.replay()
+            triton_mla.mla_decode(*call(1)[0], **call(1)[1])
+        torch.cuda.synchronize()
+        assert torch.equal(g_out, fresh[2][0]) and torch.equal(g_lse, fresh[2][1])

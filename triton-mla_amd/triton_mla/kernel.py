@@ -444,8 +444,12 @@ def mla_decode(
         num_heads] float32).
     """
     single = DEFAULT_SINGLE_LAUNCH if single_launch is None else bool(single_launch)
-    if not single and kv_scale is None:
-        res = _fast_call(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, return_lse)
+    if not single:
+        if kv_scale is None and q.dim() == 3 and q.dtype != torch.float32 and head_dim_v == 512 and q.shape[-1] == 576:
+            res = _fast_call(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, return_lse)
+        else:
+            res = _fast_call_other(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits,
+                                   kv_scale)
         if res is not None:
             return res if return_lse else res[0]
     if q.dtype == torch.float32 or head_dim_v != 512 or q.shape[-1] != 576:
@@ -478,7 +482,8 @@ def _generic_splits(batch, num_heads, capacity, num_sms, heads_per_wg=16):
     return max(1, min(by_cus, by_len, 65535))
 
 
-def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, return_lse):
+def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, return_lse,
+                    learn=None):
     """``mla_decode`` at head dims or an element type the matrix-core kernels
     are not built for (tmla_mla_decode_generic): any power-of-two head_dim_v
     in [16, 1024] and rope_dim in [16, 256], bf16, fp16 or fp32 -- the
@@ -550,20 +555,22 @@ def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax
         if block_table is not None and num_blocks == 0:
             raise ValueError("kv_cache holds no pages")
         if workers:
-            fn, parts = lib.tmla_mla_decode_generic_balanced, workers
+            name, parts = "tmla_mla_decode_generic_balanced", workers
             ws_bytes = lib.tmla_generic_balanced_workspace_bytes(batch, num_heads, head_dim_v, workers)
         else:
-            fn, parts = lib.tmla_mla_decode_generic, num_splits
+            name, parts = "tmla_mla_decode_generic", num_splits
             ws_bytes = lib.tmla_generic_workspace_bytes(batch, num_heads, head_dim_v, num_splits)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
         dev_idx = device.index if device.index is not None else torch.cuda.current_device()
-        with _OnDevice(dev_idx):
-            _native.check(fn(
-                q.data_ptr(), q.stride(0), q.stride(1), kv_cache.data_ptr(), kv_cache.stride(0), kv_cache.stride(1),
+        args = (q.data_ptr(), q.stride(0), q.stride(1), kv_cache.data_ptr(), kv_cache.stride(0), kv_cache.stride(1),
                 num_blocks, page_size, *bt_args, cache_seqlens.data_ptr(), batch, num_heads, head_dim_v, d_rope,
                 dtype, float(softmax_scale), parts, out.data_ptr(), out.stride(0), out.stride(1), lse.data_ptr(),
-                workspace.data_ptr(), ws_bytes, torch.cuda.current_stream(device).cuda_stream),
-                "tmla_mla_decode_generic")
+                workspace.data_ptr(), ws_bytes)
+        if learn is not None:
+            learn.set(name, args, dev_idx, out, lse, ws_bytes,
+                      q=0, kv=3, bt=8 if block_table is not None else None, seqlens=11, out_at=19, lse_at=22, ws_at=23)
+        with _OnDevice(dev_idx):
+            _native.check(getattr(lib, name)(*args, torch.cuda.current_stream(device).cuda_stream), name)
     if return_lse:
         return out, lse
     return out
@@ -692,3 +699,110 @@ def _shape_of(call, dtype):
         shape.plan = shape.fast.plan(*shape.a_q, *shape.a_kv, *shape.a_bt, *shape.a_mid, *shape.a_out,
                                      shape.ws_bytes)
     return shape
+
+
+class _OtherShape:
+    """The kept shape of an fp8, multi-token or generic call: its C entry, the
+    constant arguments, and where this call's addresses go among them."""
+
+    __slots__ = ("dev_idx", "device", "fn", "name", "args", "out_shape", "lse_shape", "ws_alloc", "at")
+
+    def set(self, name, args, dev_idx, out, lse, ws_bytes, q, kv, bt, seqlens, out_at, lse_at, ws_at, scale=None):
+        self.name, self.args, self.dev_idx, self.device = name, list(args), dev_idx, out.device
+        self.fn = getattr(_native.load_gil_held(), name)
+        self.out_shape, self.lse_shape = tuple(out.shape), tuple(lse.shape)
+        self.ws_alloc = max(ws_bytes, 1)
+        self.at = (q, kv, bt, seqlens, out_at, lse_at, ws_at, scale)
+
+
+_OTHER_SHAPES = {}
+_PLAIN_NUMBERS = {int, float, type(None)}
+
+
+def _fast_call_other(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, kv_scale):
+    """(out, lse) of an fp8, multi-token or generic call, or None to take the
+    full path: the first call of a shape runs that path, which validates it,
+    and keeps its constant arguments where no argument had to be copied or
+    converted; later ones only read addresses and allocate the outputs (before,
+    such calls took 25 us each however small, host time alone; with the kept
+    arguments fp8, multi-token and generic calls of one or two short sequences
+    take 14 to 15.5 us). The workspace is the stream's (see _STREAM_WS): these entries'
+    kernels too write every workspace byte they read."""
+    try:
+        key = (q.shape, q.stride(), q.dtype, q.get_device(), kv_cache.shape, kv_cache.stride(), kv_cache.dtype,
+               kv_cache.get_device(), cache_seqlens.dtype, cache_seqlens.get_device(), cache_seqlens.shape,
+               cache_seqlens.stride(),
+               None if block_table is None else (block_table.dtype, block_table.get_device(), block_table.shape,
+                                                 block_table.stride()),
+               None if kv_scale is None else (kv_scale.dtype, kv_scale.get_device(), kv_scale.shape, kv_scale.stride()),
+               head_dim_v, softmax_scale, num_splits)
+    except (AttributeError, TypeError):
+        return None
+    # plain tensors and numbers only: a tensor as the scale would be compared by
+    # identity, and a subclass of Tensor would hand its type on to the outputs
+    if type(q) is not torch.Tensor or not {type(x) for x in (head_dim_v, softmax_scale, num_splits)} <= _PLAIN_NUMBERS:
+        return None
+    qp, kp = q.data_ptr(), kv_cache.data_ptr()
+    if (qp | kp) & 15 or not qp or not kp:
+        return None
+    shape = _OTHER_SHAPES.get(key)
+    if shape is None:
+        return _learn_other(key, q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits,
+                            kv_scale)
+    if not shape or _current_device() != shape.dev_idx:
+        return None
+    out = q.new_empty(shape.out_shape)
+    lse = q.new_empty(shape.lse_shape, dtype=torch.float32)
+    stream = _raw_stream(shape.dev_idx)
+    ws, wsp = _workspace(shape, stream)
+    iq, ikv, ibt, isl, iout, ilse, iws, isc = shape.at
+    args = shape.args.copy()
+    args[iq], args[ikv], args[isl] = qp, kp, cache_seqlens.data_ptr()
+    args[iout], args[ilse], args[iws] = out.data_ptr(), lse.data_ptr(), wsp
+    if ibt is not None:
+        args[ibt] = block_table.data_ptr()
+    if isc is not None:
+        args[isc] = kv_scale.data_ptr()
+    status = shape.fn(*args, stream)
+    if status:
+        _native.check(status, shape.name)
+    return out, lse
+
+
+def _learn_other(key, q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, kv_scale):
+    """Run one call of a new shape through the full path and keep what
+    _fast_call_other needs; False (kept too) where an argument was copied or
+    converted. Returns the call's (out, lse), or None for a shape not kept."""
+    plain = (q.get_device() >= 0 and kv_cache.get_device() == q.get_device()
+             and cache_seqlens.dtype == torch.int32 and cache_seqlens.get_device() == q.get_device()
+             and cache_seqlens.is_contiguous()
+             and (block_table is None or (block_table.dtype == torch.int32 and block_table.get_device() == q.get_device()
+                                          and block_table.dim() == 2 and block_table.stride(-1) == 1))
+             and (kv_scale is None or (kv_scale.dtype == torch.float32 and kv_scale.get_device() == q.get_device()
+                                       and kv_scale.is_contiguous()))
+             and q.dim() in (3, 4) and q.shape[0] > 0 and q.stride(-1) == 1)
+    shape, res = _OtherShape(), None
+    if plain and (q.dtype == torch.float32 or head_dim_v != 512 or q.shape[-1] != 576):
+        if kv_scale is None and q.dim() == 3:
+            res = _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, True,
+                                  learn=shape)
+    elif plain and (q.dim() == 3 or q.stride(1) == q.shape[2] * q.stride(2)):
+        call = DecodeLaunch(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits,
+                            kv_scale=kv_scale)
+        res = call.run(False)
+        kept = call._keep
+        if kept[0].data_ptr() == q.data_ptr() and kept[1].data_ptr() == kv_cache.data_ptr() \
+                and (kv_scale is None or kept[4].data_ptr() == kv_scale.data_ptr()):
+            bt = 8 if block_table is not None else None
+            if call.fp8:  # the scale pointer at 8, q_len after 13 + 3 arguments
+                shape.set("tmla_mla_decode_fp8", call._fp8_args, call._dev_idx, call.out, call.lse, call.ws_bytes, q=0,
+                          kv=3, bt=None if bt is None else 11, seqlens=14, out_at=24, lse_at=27, ws_at=28, scale=8)
+            elif call.q_len > 1:  # q_len at 13, the single-launch flag last
+                shape.set("tmla_mla_decode_causal", call._causal_args + (0,), call._dev_idx, call.out, call.lse,
+                          call.ws_bytes, q=0, kv=3, bt=bt, seqlens=11, out_at=21, lse_at=24, ws_at=25)
+    if len(_OTHER_SHAPES) > 1024:
+        _OTHER_SHAPES.clear()
+    # (a workspace past 256 MiB is not kept beyond its call)
+    keep = getattr(shape, "args", None) is not None and shape.ws_alloc <= 256 << 20
+    _OTHER_SHAPES[key] = shape if keep else False
+    return res
