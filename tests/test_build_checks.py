@@ -1,14 +1,17 @@
 """The checks triton-mla_amd/build.py runs on every build, on planted inputs:
-the resource-report parser and its scratch/LDS gate, and the scan for reads
-of an inline-asm MFMA result before the MFMA has finished. (The real build
-runs them on the shipped code; here each must catch what it is for.)"""
+the resource-report parser and its scratch/LDS gate, and the scans for the
+hazards of inline asm. (The real build runs them on the shipped code; here each
+must catch what it is for.)"""
 
 import os
+import re
+import subprocess
 import sys
 
 import pytest
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "triton-mla_amd"))
+import asm_checks  # noqa: E402
 import build  # noqa: E402
 
 REMARKS = """\
@@ -69,3 +72,84 @@ def test_mfma_hazard_scan(tmp_path):
     # MFMAs into AGPRs are the compiler's own (it inserts their waits)
     agpr = "\tv_mfma_f32_32x32x16_bf16 a[0:15], v[32:35], v[36:39], a[0:15]\n"
     assert build.mfma_result_hazards(_asm(tmp_path, agpr + "\tv_mov_b32_e32 v60, v7\n")) == []
+
+
+def _in_asm(body):
+    return "\t;;#ASMSTART\n" + body + "\t;;#ASMEND\n"
+
+
+def test_mfma_result_scan_follows_branches(tmp_path):
+    mfma = "\tv_mfma_f32_32x32x16_bf16 v[0:15], v[32:35], v[36:39], v[0:15]\n"
+    early = "\tv_max_f32_e32 v40, v3, v40\n"
+    # one path to the read comes straight from the MFMA, the other waits
+    body = ("\ts_cbranch_scc0 .LBB0_2\n.LBB0_1:\n" + mfma + "\ts_branch .LBB0_3\n.LBB0_2:\n\ts_nop 7\n.LBB0_3:\n" +
+            early + "\ts_endpgm\n")
+    assert len(build.mfma_result_hazards(_asm(tmp_path, body))) == 1
+    # around a loop: the MFMA at the end of one turn, the read at the start of the next
+    body = ".LBB0_1:\n" + early + mfma + "\ts_cbranch_scc1 .LBB0_1\n\ts_endpgm\n"
+    assert len(build.mfma_result_hazards(_asm(tmp_path, body))) == 1
+    # an AGPR result of an inline-asm MFMA is nobody else's to wait for
+    agpr = "\tv_mfma_f32_32x32x16_bf16 a[0:15], v[32:35], v[36:39], a[0:15]\n"
+    read = "\tv_accvgpr_read_b32 v60, a7\n"
+    assert len(build.mfma_result_hazards(_asm(tmp_path, _in_asm(agpr) + read))) == 1
+    assert build.mfma_result_hazards(_asm(tmp_path, agpr + read)) == []
+
+
+def test_mfma_operand_scan(tmp_path):
+    mfma = _in_asm("\tv_mfma_f32_32x32x16_bf16 v[2:17], v[222:225], v[22:25], v[2:17]\n")
+    back = "\tv_accvgpr_read_b32 v24, a132\n"
+    other = "\tv_add_u32_e32 v100, v101, v102\n"
+
+    def hits(body):
+        return len(build.mfma_operand_hazards(_asm(tmp_path, body + "\ts_endpgm\n")))
+
+    # an operand brought back from an AGPR right before, or one instruction before
+    assert hits(back + mfma) == 1 and hits(back + other + mfma) == 1
+    assert hits(back + other + other + mfma) == 0 and hits(back + "\ts_nop 1\n" + mfma) == 0
+    assert hits(back + "\ts_nop 0\n" + mfma) == 1
+    # the accumulator is an operand too; reads of the registers and writes of others are not
+    assert hits("\tv_mov_b32_e32 v5, 0\n" + mfma) == 1
+    assert hits("\tv_add_u32_e32 v100, v24, v222\n" + mfma) == 0
+    # the compiler's own MFMA, whose waits it inserts
+    assert hits(back + mfma.replace("\t;;#ASMSTART\n", "")) == 0
+    # before a branch, and in one of two predecessors
+    assert hits(back + "\ts_cbranch_scc0 .LBB0_1\n" + other + ".LBB0_1:\n" + mfma) == 1
+    # both registers of a swap are written
+    assert hits("\tv_permlane32_swap_b32 v60, v223\n" + mfma) == 1
+
+
+def test_inline_asm_mfmas_keep_their_distance(tmp_path):
+    """Every inline-asm MFMA of the kernels starts with the two wait states an
+    operand written by the vector ALU needs (but for the head-owner loop's,
+    which the scan alone guards), and in compiled code they satisfy the scan."""
+    csrc, bare = os.path.join(os.path.dirname(build.__file__), "csrc"), []
+    for name in sorted(os.listdir(csrc)):
+        with open(os.path.join(csrc, name)) as f:
+            text = re.sub(r"//.*", "", f.read())
+        for m in re.finditer(r"\basm(?: volatile)?\(\s*([^:]*v_mfma[^:]*):", text):
+            if not m.group(1).startswith("TMLA_MFMA_GAP "):
+                bare.append(re.findall(r"__forceinline__ \w+ (\w+)\(", text[:m.start()])[-1])
+    assert sorted(bare) == ["own_mfma_acc", "own_mfma_acc", "own_mfma_first", "own_mfma_first"]
+
+    probe = """
+#include "cdna.h"
+using namespace tmla;
+__global__ void k(const i16x8* a, const i16x8* b, f32x16* o, short x) {
+  f32x16 d = o[threadIdx.x];
+  const i16x8 u = a[threadIdx.x] ^ (i16x8)x, v = b[threadIdx.x] ^ (i16x8)x;
+  asm volatile(GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(u), "v"(v));
+  asm volatile("s_nop 7\\n\\ts_nop 7\\n\\ts_nop 7" : "+v"(d));
+  o[threadIdx.x] = d;
+}
+"""
+    src = tmp_path / "probe.hip"
+    src.write_text(probe)
+    found = []
+    for gap in ("", "TMLA_MFMA_GAP"):
+        out = tmp_path / "probe.s"
+        subprocess.run([build.hipcc()] + build.FLAGS + [f"-I{csrc}", f"-DGAP={gap}", "-S", "--cuda-device-only",
+                                                        str(src), "-o", str(out)], check=True, capture_output=True)
+        assert any(ins.asm and ins.op.startswith("v_mfma") for _, blocks in asm_checks.kernels(str(out))
+                   for blk in blocks for ins in blk.ins)
+        found.append(len(asm_checks.mfma_operand_hazards(str(out))))
+    assert found[0] > 0 and found[1] == 0

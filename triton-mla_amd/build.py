@@ -14,10 +14,8 @@ linked. Every build checks the code it ships:
   * the compiler's resource report of every kernel: no scratch (register
     spills to memory) beyond the per-kernel allowances below, LDS within the
     160 KiB of a compute unit;
-  * the device assembly: no instruction reads the result registers of an
-    inline-asm MFMA before the MFMA has finished (the compiler does not know
-    the latency of inline asm, so it cannot insert the wait itself; this
-    catches a register-allocator copy of an accumulator still in flight);
+  * the device assembly: the hazards of inline asm, which the compiler does
+    not look inside and so leaves to this check (asm_checks.py);
   * the host launch stubs of every kernel are defined.
 """
 
@@ -31,6 +29,8 @@ import sys
 import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
+
+from asm_checks import mfma_operand_hazards, mfma_result_hazards
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -60,10 +60,10 @@ SCRATCH_ALLOWANCE = {
     r"mla_partial_kernelILi[01]ELi512ELi64ELi4ELb1ELb1ELb1E": 12,
 }
 
-# Cycles an inline-asm v_mfma_f32_32x32x16 result takes: instructions that
-# read or overwrite its destination must come at least this many
-# instructions (or s_nop wait states) later.
-MFMA_RESULT_WINDOW = 18
+ASM_CHECKS = {
+    "an inline-asm MFMA result touched before it is ready": mfma_result_hazards,
+    "an inline-asm MFMA operand written too shortly before it": mfma_operand_hazards,
+}
 
 
 def hipcc() -> str:
@@ -104,10 +104,11 @@ def build(verbose: bool = False, stamps: bool = False) -> str:
         usage = {}
         for remarks, asm in results:
             usage.update(parse_resource_usage(remarks))
-            bad = mfma_result_hazards(asm)
-            if bad:
-                raise RuntimeError(f"{os.path.basename(asm)}: {len(bad)} reads of an inline-asm MFMA result before "
-                                   f"it is ready, first: {bad[0][0]}  ->  {bad[0][1]}")
+            for what, scan in ASM_CHECKS.items():
+                bad = scan(asm)
+                if bad:
+                    raise RuntimeError(f"{os.path.basename(asm)}: {len(bad)} of {what}, first: "
+                                       f"{bad[0][0]}  ->  {bad[0][1]}")
         # the profiling build's stamp code takes registers of its own: its
         # scratch is reported, not refused
         check_resources(usage, strict=not stamps)
@@ -122,7 +123,7 @@ def build(verbose: bool = False, stamps: bool = False) -> str:
         build_fast_ext()
     if verbose:
         print(f"{len(usage)} kernels checked" + ("" if stamps else ", none beyond their scratch allowance") +
-              ", no early MFMA result reads", flush=True)
+              ", no hazards of inline asm", flush=True)
     return out
 
 
@@ -181,60 +182,6 @@ def check_resources(usage: dict[str, dict[str, int]], strict: bool = True) -> No
             problems.append(f"{name}: {u['LDS Size']} bytes of LDS")
     if problems:
         raise RuntimeError("kernel resources:\n  " + "\n  ".join(problems))
-
-
-def _vregs(operand: str) -> set[int]:
-    regs = set()
-    for m in re.finditer(r"\bv\[(\d+):(\d+)\]", operand):
-        regs |= set(range(int(m.group(1)), int(m.group(2)) + 1))
-    for m in re.finditer(r"\bv(\d+)\b", operand):
-        regs.add(int(m.group(1)))
-    return regs
-
-
-def mfma_result_hazards(asm_path: str, window: int = MFMA_RESULT_WINDOW) -> list[tuple[str, str]]:
-    """(MFMA, reader) pairs in which an instruction touches the VGPR result of
-    an MFMA fewer than ``window`` instructions (s_nop counts its wait states)
-    after it. MFMAs with an AGPR result are the compiler's own (it inserts
-    their waits); one MFMA accumulating into the exact result of the previous
-    one is the hardware's back-to-back case and allowed. Straight-line code
-    only: the window restarts at every label."""
-    bad = []
-    pending: list[tuple[set[int], int, str]] = []  # (result VGPRs, instructions left, MFMA)
-    with open(asm_path) as f:
-        for raw in f:
-            t = raw.split(";")[0].strip()
-            if not t or t.startswith("."):
-                continue
-            if t.endswith(":"):
-                pending = []
-                continue
-            op, _, args = t.partition(" ")
-            parts = [p.strip() for p in args.split(",")] if args else []
-            if op.startswith("s_nop"):
-                n = (int(parts[0], 0) if parts and parts[0] else 0) + 1
-                pending = [(r, w - n, x) for r, w, x in pending if w - n > 0]
-                continue
-            if op.startswith("v_mfma") and len(parts) >= 4 and parts[0].startswith("v"):
-                dst, src_c = _vregs(parts[0]), _vregs(parts[3])
-                src_ab = _vregs(parts[1]) | _vregs(parts[2])
-                for r, _, x in pending:
-                    if (src_ab | src_c) & r and not (src_c == r and not src_ab & r):
-                        bad.append((x, t))
-                pending = [(r, w - 1, x) for r, w, x in pending if w - 1 > 0 and not r & dst]
-                pending.append((dst, window, t))
-                continue
-            stores = op.startswith(("ds_write", "global_store", "buffer_store", "scratch_store"))
-            touched = set()
-            for p in (parts if stores else parts[1:]):
-                touched |= _vregs(p)
-            if parts and not stores:
-                touched |= _vregs(parts[0])
-            for r, _, x in pending:
-                if touched & r:
-                    bad.append((x, t))
-            pending = [(r, w - 1, x) for r, w, x in pending if w - 1 > 0]
-    return bad
 
 
 def check_kernel_stubs(path: str) -> None:

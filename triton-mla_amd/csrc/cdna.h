@@ -49,6 +49,15 @@ __device__ __forceinline__ i16x8 ds_read_b128(const char LDS_AS* p) {
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(p), "i"(OFF));
   return r;
 }
+
+// Put before an MFMA written as inline asm. An MFMA may read a register only
+// two wait states after a vector-ALU instruction wrote it; the compiler keeps
+// to that for its own MFMAs but does not look inside asm, and it may place
+// such a write (a Q^T operand brought back from an AGPR, say) right before
+// any asm statement: which builds have one is up to the register allocator.
+// (own_mfma_first / own_mfma_acc in mla_decode.hip go without.)
+#define TMLA_MFMA_GAP "s_nop 1\n\t"
+
 // One LDS-DMA copy: 16 bytes per lane from src + OFF into LDS at
 // dst + 16 * lane (global_load_lds_dwordx4; completion counts in vmcnt). The
 // instruction's immediate offset applies to both addresses, so the LDS base

@@ -268,20 +268,24 @@ constexpr int pass_reads(int t) {
 
 // S^T accumulation in VGPRs (the PV accumulators own every AGPR). After the
 // chain, mfma_vgpr_fence waits out the MFMA result latency before any VALU
-// instruction reads the accumulator.
+// instruction reads the accumulator. (TMLA_MFMA_GAP costs the fp8 ring at 32
+// sequences of 8K tokens and 128 heads 97.9 -> 99.1 us. Without it, a build
+// whose single launch merged with the combine's functions brought a Q^T
+// operand back from AGPRs right before its MFMA in the 32-head fp8 instance
+// and gave wrong scores.)
 template <int DT>
 __device__ __forceinline__ f32x16 mfma_vgpr_first(const i16x8& a, const i16x8& b) {
   f32x16 d;
   if constexpr (TMLA_MFMA_VOLATILE) {
     if constexpr (DT == TMLA_BF16)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
     else
-      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
   } else {
     if constexpr (DT == TMLA_BF16)
-      asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
+      asm(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
     else
-      asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
+      asm(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(b));
   }
   return d;
 }
@@ -289,14 +293,14 @@ template <int DT>
 __device__ __forceinline__ void mfma_vgpr_acc(f32x16& d, const i16x8& a, const i16x8& b) {
   if constexpr (TMLA_MFMA_VOLATILE) {
     if constexpr (DT == TMLA_BF16)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
     else
-      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
   } else {
     if constexpr (DT == TMLA_BF16)
-      asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+      asm(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
     else
-      asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+      asm(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
   }
 }
 // O^T += V^T . P^T with the accumulator in AGPRs. The volatile asm form
@@ -308,9 +312,9 @@ template <int DT>
 __device__ __forceinline__ void mfma_agpr_acc(f32x16& acc, const i16x8& v, const i16x8& p) {
   if constexpr (TMLA_MFMA_VOLATILE) {
     if constexpr (DT == TMLA_BF16)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
     else
-      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+      asm volatile(TMLA_MFMA_GAP "v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
   } else {
     acc = Elt<DT>::mfma(v, p, acc);
     asm volatile("" : "+a"(acc));
@@ -1478,7 +1482,12 @@ void mla_partial_kernel(PartialArgs a) {
 // S^T MFMAs of the head-owner loop: volatile asm, so they keep their places
 // among the operand reads and waits and keep their accumulators in VGPRs
 // (the value accumulators own every AGPR). The VALU reads of their results
-// are placed a fixed number of steps later, past the result latency.
+// are placed a fixed number of steps later, past the result latency. Without
+// TMLA_MFMA_GAP: two cycles before each of the 36 MFMAs of a sub-tile cost
+// this loop, bound by instruction issue, 1.9% (64 sequences of 1K to 32K tokens,
+// 128 heads: 343 us without, 350 with). Its operands come straight from LDS
+// reads or stay in VGPRs, and build.py refuses a build in which one is written
+// by a vector-ALU instruction too shortly before its MFMA.
 template <int DT>
 __device__ __forceinline__ f32x16 own_mfma_first(const i16x8& a, const i16x8& b) {
   f32x16 d;

@@ -104,13 +104,13 @@ struct F8Elt<TMLA_BF16> {
   }
   // (asm: see the note on MFMA forms below)
   __device__ static __forceinline__ void mfma_qk_first(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_qk(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_pv(f32x4& acc, const v4& v, const v4& p) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
   }
   __device__ static __forceinline__ __bf16 round(float x) { return (__bf16)x; }
 };
@@ -123,13 +123,13 @@ struct F8Elt<TMLA_FP16> {
     return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, 1.0f, HI);
   }
   __device__ static __forceinline__ void mfma_qk_first(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_qk(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_pv(f32x4& acc, const v4& v, const v4& p) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
   }
   __device__ static __forceinline__ _Float16 round(float x) { return (_Float16)x; }
 };

@@ -84,13 +84,13 @@ struct Elt16<TMLA_BF16> {
   typedef bf16x8 v8;
   typedef bf16x4 v4;
   __device__ static __forceinline__ void mfma_qk_first(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_qk(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_pv(f32x4& acc, const v4& v, const v4& p) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
   }
   __device__ static __forceinline__ __bf16 round(float x) { return (__bf16)x; }
 };
@@ -99,13 +99,13 @@ struct Elt16<TMLA_FP16> {
   typedef f16x8 v8;
   typedef f16x4 v4;
   __device__ static __forceinline__ void mfma_qk_first(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_qk(f32x4& d, const v8& k, const v8& q) {
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(d) : "v"(k), "v"(q));
   }
   __device__ static __forceinline__ void mfma_pv(f32x4& acc, const v4& v, const v4& p) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
+    asm volatile(TMLA_MFMA_GAP "v_mfma_f32_16x16x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(v), "v"(p));
   }
   __device__ static __forceinline__ _Float16 round(float x) { return (_Float16)x; }
 };
