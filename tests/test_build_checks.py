@@ -118,6 +118,37 @@ def test_mfma_operand_scan(tmp_path):
     assert hits("\tv_permlane32_swap_b32 v60, v223\n" + mfma) == 1
 
 
+def test_inflight_load_scan(tmp_path):
+    read = _in_asm("\tds_read_b128 v[54:57], v2 offset:0\n")
+    more = _in_asm("\tds_read_b64_tr_b16 v[60:61], v3 offset:0\n")
+    scalar = _in_asm("\ts_load_dword s30, s[98:99], 0x0\n")
+    copy, scopy = "\tv_mov_b64_e32 v[70:71], v[56:57]\n", "\ts_mov_b32 s10, s30\n"
+
+    def wait(n):
+        return f"\ts_waitcnt lgkmcnt({n})\n"
+
+    def hits(body):
+        return len(build.inflight_touches(_asm(tmp_path, body + "\ts_endpgm\n")))
+
+    # copied, overwritten (its value unused) or loaded again before it has arrived
+    assert hits(read + copy) == 1 and hits(read + "\tv_mov_b32_e32 v55, 0\n") == 1 and hits(read + read) == 1
+    assert hits(read + wait(0) + copy) == 0
+    # a counted wait covers all but the newest reads and writes of LDS
+    assert hits(read + more + wait(1) + copy) == 0 and hits(read + more + wait(2) + copy) == 1
+    assert hits(read + "\tds_write_b32 v4, v5\n" + wait(1) + copy) == 0
+    assert hits(more + read + wait(1) + copy) == 1
+    # ... but a scalar load is covered by none but zero, and covers no LDS read
+    assert hits(scalar + scopy) == 1 and hits(scalar + more + wait(1) + scopy) == 1
+    assert hits(scalar + more + wait(0) + scopy) == 0 and hits(read + scalar + wait(1) + copy) == 1
+    # a wait in one of two branches only, and around a loop
+    branch = "\ts_cbranch_scc0 .LBB0_1\n" + wait(0) + ".LBB0_1:\n"
+    assert hits(read + branch + copy) == 1 and hits(read + wait(0) + branch + copy) == 0
+    assert hits(".LBB0_1:\n" + scopy + scalar + "\ts_cbranch_scc1 .LBB0_1\n") == 1
+    # a wait for other counters; the compiler's own loads, which it waits for
+    assert hits(read + "\ts_waitcnt vmcnt(0)\n" + copy) == 1
+    assert hits("\tds_read_b128 v[54:57], v2\n" + copy) == 0
+
+
 def test_inline_asm_mfmas_keep_their_distance(tmp_path):
     """Every inline-asm MFMA of the kernels starts with the two wait states an
     operand written by the vector ALU needs (but for the head-owner loop's,

@@ -1,17 +1,22 @@
 """Scans of the compiler's gfx950 assembly for hazards of inline asm.
 
 The compiler inserts the waits and wait states that its own instructions
-need, but it does not look inside inline asm. Two things can therefore go
+need, but it does not look inside inline asm. Three things can therefore go
 wrong without any message, depending on nothing but the register allocation
 of one build:
 
+  * ``inflight_touches``: the destination of an LDS or scalar load issued by
+    inline asm is read, copied or overwritten before an ``s_waitcnt lgkmcnt``
+    that covers it (LDS operations return in order, so ``lgkmcnt(n)`` covers
+    all but the newest n; scalar loads return in any order and are covered by
+    ``lgkmcnt(0)`` only);
   * ``mfma_operand_hazards``: a vector-ALU instruction (a copy out of an AGPR
     for instance) writes an operand of an inline-asm MFMA fewer than two wait
     states before it;
   * ``mfma_result_touches``: the result of an MFMA is read or overwritten
     before the MFMA has finished, where one of the two is inline asm.
 
-Both follow every branch of a kernel (a forward dataflow analysis over
+All three follow every branch of a kernel (a forward dataflow analysis over
 its blocks, taking the worst of all paths that lead to a block, whatever the
 branch conditions). An instruction counts as one wait state, ``s_nop n`` as
 n + 1.
@@ -24,6 +29,7 @@ from typing import NamedTuple
 
 OPERAND_WAIT_STATES = 2  # vector-ALU write of a register -> MFMA that reads it
 RESULT_WINDOW = 18       # wait states after which any MFMA used here has finished
+_COUNTER = 15            # lgkmcnt counts to 15
 
 _REG = re.compile(r"\b([vsa])(?:\[(\d+):(\d+)\]|(\d+))(?![\w\[])")
 
@@ -36,6 +42,7 @@ class Ins(NamedTuple):
     asm: bool  # issued by inline asm
     text: str
     nop: int  # wait states it takes
+    wait: int  # lgkmcnt it waits for (-1: none)
     target: str  # branch target, "" for none
 
 
@@ -58,8 +65,12 @@ def _parse(text: str):
                 regs.update((kind, i) for i in (range(int(lo), int(hi) + 1) if lo else (int(one),)))
             parts.append(frozenset(regs))
         nop = int(args.strip(), 0) + 1 if op == "s_nop" else 1
+        wait = -1
+        if op == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", args)
+            wait = int(m.group(1)) if m else 0 if args.strip() == "0" else -1
         target = args.split()[-1] if op.startswith(("s_cbranch", "s_branch")) else ""
-        got = _parsed[text] = (op, tuple(parts), frozenset().union(*parts), nop, target)
+        got = _parsed[text] = (op, tuple(parts), frozenset().union(*parts), nop, wait, target)
     return got
 
 
@@ -89,8 +100,8 @@ def kernels(asm_path: str):
                 continue
             if t.startswith(".") or name is None:
                 continue
-            op, parts, regs, nop, target = _parse(re.sub(r"\s+", " ", t))
-            body.append(Ins(ln, op, parts, regs, in_asm, t, nop, target))
+            op, parts, regs, nop, wait, target = _parse(re.sub(r"\s+", " ", t))
+            body.append(Ins(ln, op, parts, regs, in_asm, t, nop, wait, target))
         if name is not None:
             yield name, _blocks(body)
 
@@ -161,6 +172,34 @@ def _scan(asm_path: str, wanted, step, merge) -> list:
         if any(wanted(ins) for blk in blocks for ins in blk.ins):
             found += _flow(blocks, step, merge)
     return found
+
+
+def _asm_load(ins: Ins) -> bool:
+    return ins.asm and ins.op.startswith(("ds_read", "s_load"))
+
+
+def inflight_touches(asm_path: str) -> list:
+    """(load, instruction) pairs: see the module's docstring."""
+
+    # register -> (LDS operations issued since its load, the load); a scalar
+    # load's count stays at -1, so that only lgkmcnt(0) covers it
+    def step(state, ins, report):
+        if ins.wait >= 0:
+            for reg in [r for r, (since, _) in state.items() if ins.wait == 0 or since >= ins.wait]:
+                del state[reg]
+            return
+        if state:
+            for reg in ins.regs & state.keys():
+                report(ins, state.pop(reg)[1])
+            if ins.op.startswith("ds_"):
+                for reg, (since, load) in state.items():
+                    if 0 <= since < _COUNTER:
+                        state[reg] = (since + 1, load)
+        if _asm_load(ins):
+            for reg in ins.parts[0]:
+                state[reg] = (0 if ins.op.startswith("ds_") else -1, ins)
+
+    return _scan(asm_path, _asm_load, step, min)
 
 
 def _asm_mfma(ins: Ins) -> bool:

@@ -30,7 +30,7 @@ import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
-from asm_checks import mfma_operand_hazards, mfma_result_hazards
+from asm_checks import inflight_touches, mfma_operand_hazards, mfma_result_hazards
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -61,6 +61,7 @@ SCRATCH_ALLOWANCE = {
 }
 
 ASM_CHECKS = {
+    "an inline-asm load's destination touched before it has arrived": inflight_touches,
     "an inline-asm MFMA result touched before it is ready": mfma_result_hazards,
     "an inline-asm MFMA operand written too shortly before it": mfma_operand_hazards,
 }
@@ -107,7 +108,7 @@ def build(verbose: bool = False, stamps: bool = False) -> str:
             for what, scan in ASM_CHECKS.items():
                 bad = scan(asm)
                 if bad:
-                    raise RuntimeError(f"{os.path.basename(asm)}: {len(bad)} of {what}, first: "
+                    raise RuntimeError(f"{os.path.basename(asm)}: {len(bad)} times {what}, first: "
                                        f"{bad[0][0]}  ->  {bad[0][1]}")
         # the profiling build's stamp code takes registers of its own: its
         # scratch is reported, not refused

@@ -1116,9 +1116,11 @@ void mla_partial_kernel(PartialArgs a) {
         next_page = i < 0 ? pro_page[kStages - 1] : page_fetch(st0 + i + kStages);
       if (F8 && do_copy) sc3 = s_load_f32(a.kv_scale + (int64_t)page * a.sc_s0);  // sub-tile i+3
       const int pbuf = i & 1;
-      // the factors of PV(i) (waves without S read them again where they use
-      // them, see pass1_hook)
-      f32x4 alpha4 = ds_read_f32x4(lds + OFF_A + pbuf * ASLOT + (lane & 31) * 16);
+      const char LDS_AS* const factors = lds + OFF_A + pbuf * ASLOT + (lane & 31) * 16;
+      // the factors of PV(i); a wave without S reads them where it uses them
+      // (see pass1_hook), so that no read's registers are left unused
+      f32x4 alpha4;
+      if (NHB == NW || s_owner) alpha4 = ds_read_f32x4(factors);
       // ring entries (i + 1 >= 0): S(i+1) reads entry i+1, PV(i) entry i
       // (entry 0 at i = -1, where P = 0), the copies fill entry i+3 (16-bit
       // cache; the fp8 widening fills entry i+2 above)
@@ -1148,12 +1150,11 @@ void mla_partial_kernel(PartialArgs a) {
           if constexpr (j == PV_START - 1) {
             // An S wave's operand waits cover the factors' read, which is
             // older than every read of the pass. A wave without S has waited
-            // for nothing yet, and its branch may copy registers of a read in
-            // flight: it reads them here and waits.
+            // for nothing yet: it reads them here and waits.
             if constexpr (NST == NKC) {
               pin_f4(alpha4);
             } else {
-              alpha4 = ds_read_f32x4(lds + OFF_A + pbuf * ASLOT + (lane & 31) * 16);
+              alpha4 = ds_read_f32x4(factors);
               lgkm_tie_f4<0>(alpha4);
             }
             bool any = false;
@@ -1285,6 +1286,13 @@ void mla_partial_kernel(PartialArgs a) {
         else
           pv_iteration();
       }
+      // The iteration's scalar loads (page id, fp8 scale) have arrived. The
+      // next iteration starts with this wait anyway; here it ties their
+      // registers before the compiler copies them on the way there.
+      if constexpr (F8)
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(next_page), "+s"(sc3));
+      else if constexpr (PAGED && PAGE_UNIFORM)
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(next_page));
     };
     // Iteration -1 always runs with copies: for a segment of fewer than
     // kStages - 1 sub-tiles its copy is of a clamped (valid) row into an
