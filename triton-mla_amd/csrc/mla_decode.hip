@@ -1286,13 +1286,15 @@ void mla_partial_kernel(PartialArgs a) {
         else
           pv_iteration();
       }
-      // The iteration's scalar loads (page id, fp8 scale) have arrived. The
-      // next iteration starts with this wait anyway; here it ties their
-      // registers before the compiler copies them on the way there.
+      // Every load of the iteration has arrived. The next one starts with this
+      // wait anyway; here it ties the registers of the scalar loads (page id,
+      // fp8 scale) before the compiler copies them on the way there.
       if constexpr (F8)
         asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(next_page), "+s"(sc3));
       else if constexpr (PAGED && PAGE_UNIFORM)
         asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(next_page));
+      else
+        asm volatile("s_waitcnt lgkmcnt(0)");
     };
     // Iteration -1 always runs with copies: for a segment of fewer than
     // kStages - 1 sub-tiles its copy is of a clamped (valid) row into an
