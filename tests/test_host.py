@@ -219,3 +219,28 @@ def test_down_projection_in_inference_mode(made_in_inference):
         q_lat, kv = layer._down_proj(xg)
         (q_lat.sum() + kv.sum()).backward()
         assert xg.grad is not None
+
+
+def test_kept_arguments_refuse_what_the_full_path_refuses(monkeypatch):
+    """A repeated call whose head_dim_v merely equals the kept one (256.0, which
+    the full path refuses) does not take the kept arguments."""
+    from triton_mla import kernel as K
+
+    class Taken(Exception):
+        pass
+
+    def taken():
+        raise Taken
+
+    q, kv, lens = torch.zeros(2, 16, 288), torch.zeros(2, 40, 288), torch.tensor([40, 20], dtype=torch.int32)
+    monkeypatch.setattr(K, "_OTHER_SHAPES", {})
+    monkeypatch.setattr(K, "_learn_other", lambda key, *args: K._OTHER_SHAPES.setdefault(key, object()) and None)
+    monkeypatch.setattr(K, "_current_device", taken)
+    assert K._fast_call_other(q, kv, lens, None, 256, None, None, None) is None and len(K._OTHER_SHAPES) == 1
+    monkeypatch.setattr(K._OtherShape, "dev_idx", 0, raising=False)
+    K._OTHER_SHAPES = {k: K._OtherShape() for k in K._OTHER_SHAPES}
+    with pytest.raises(Taken):
+        K._fast_call_other(q, kv, lens, None, 256, None, None, None)
+    assert K._fast_call_other(q, kv, lens, None, 256.0, None, None, None) is None
+    with pytest.raises(AttributeError):  # the full path's refusal
+        K.mla_decode(q, kv, lens, head_dim_v=256.0)

@@ -739,8 +739,10 @@ def _fast_call_other(q, kv_cache, cache_seqlens, block_table, head_dim_v, softma
     except (AttributeError, TypeError):
         return None
     # plain tensors and numbers only: a tensor as the scale would be compared by
-    # identity, and a subclass of Tensor would hand its type on to the outputs
-    if type(q) is not torch.Tensor or not {type(x) for x in (head_dim_v, softmax_scale, num_splits)} <= _PLAIN_NUMBERS:
+    # identity, a subclass of Tensor would hand its type on to the outputs, and
+    # 512.0, which the full path refuses as head_dim_v, equals a kept 512
+    if type(q) is not torch.Tensor or type(head_dim_v) is not int \
+            or not {type(x) for x in (softmax_scale, num_splits)} <= _PLAIN_NUMBERS:
         return None
     qp, kp = q.data_ptr(), kv_cache.data_ptr()
     if (qp | kp) & 15 or not qp or not kp:
