@@ -3,10 +3,13 @@
 // sanitizers (any signed overflow, out-of-range shift or bad access aborts).
 // It sweeps extreme batch, head, split, worker and capacity values through
 // check_common, ws_layout, worker_grid, plan_launch and plan_launch_g16, and the
-// generic decode's check_generic, generic_plan and generic_workspace_bytes, and checks
+// generic decode's check_generic, generic_plan, generic_workspace_bytes, token look-ahead and balanced
+// form (dims_form, dims_workers, generic_balanced_workspace_bytes), and checks
 // the invariants the kernels rely on. Prints "ok <cases>" on success.
 #include <stdio.h>
 #include <stdlib.h>
+
+#include <initializer_list>
 
 #include "host_plan.h"
 
@@ -135,6 +138,58 @@ int main() {
                 }
               }
       }
+  // the balanced generic form: heads per workgroup, workers, workspace, grid
+  for (int32_t dv : gdims)
+    for (int32_t dr : gdims) {
+      const bool form = dims_form(dv, dr);
+      EXPECT(!form || (dv % 64 == 0 && dv <= 512 && dr % 16 == 0 && dr <= 64), "form dv=%d dr=%d", dv, dr);
+      if (!form) continue;
+      for (int dt = 0; dt <= 2; ++dt)
+        for (int32_t h : {1, 16, 17, 32, 33, 128, 129, 65535, I32})
+          for (int cus : cus_list) {
+            ++cases;
+            const int32_t per = dims_heads_per_workgroup(dt, h);
+            EXPECT(dt == TMLA_FP32 ? (per == 16 || per == 32) && (h > 16) == (per == 32) : per == 128, "per %d", per);
+            const int32_t w = dims_workers(dv, dt, h, cus);
+            const int64_t gy = ((int64_t)h + per - 1) / per;
+            EXPECT(w >= 1 && w <= 2 * cus, "workers %d cus=%d", w, cus);
+            EXPECT(w == 1 || w * gy <= (int64_t)cus * (dt == TMLA_FP32 && dv <= 256 ? 2 : 1), "one round h=%d", h);
+          }
+    }
+  for (int32_t b : gbatches)
+    for (int32_t h : gheads)
+      for (int32_t w : {-1, 0, 1, 256, 65535, I32})
+        for (int32_t dv : {64, 128, 256, 512}) {
+          ++cases;
+          const size_t need = generic_balanced_workspace_bytes(b, h, dv, w);
+          const int64_t slots = (int64_t)b + w;
+          if (h <= 0 || w <= 0 || slots > I32) {
+            EXPECT(need == 0, "balanced need b=%d h=%d w=%d", b, h, w);
+            continue;
+          }
+          // (rows of the call, and their lse at the next 256-byte boundary)
+          const int64_t rows = slots * h;
+          const bool fits = rows <= kMaxWorkspaceBytes / ((int64_t)dv + 1) / 4 - 256;
+          EXPECT(fits == (need > 0), "balanced fits b=%d h=%d w=%d", b, h, w);
+          if (need > 0) EXPECT((int64_t)need >= rows * ((int64_t)dv + 1) * 4 && need % 256 == 0, "balanced need");
+          for (int64_t cap : caps) {
+            const int64_t g = worker_grid(b, 0, w, cap);
+            EXPECT(g >= 1 && g <= w, "balanced grid b=%d w=%d cap=%lld", b, w, (long long)cap);
+          }
+        }
+  // copies past a piece's end: pieces [first, end) of the longest lengths, up
+  // to four 64-token steps past it
+  for (int32_t end : {1, 63, 64, 65, 1 << 20, kMaxGenericLen - 63, kMaxGenericLen})
+    for (int64_t first : {(int64_t)0, (int64_t)end / 2 / 64 * 64, ((int64_t)end - 1) / 64 * 64})
+      for (int64_t t = end > 300 ? end - 300 : first; t < (int64_t)end + 256; ++t)
+        for (uint32_t n : {1u, 32u}) {
+          if (t < first) continue;
+          ++cases;
+          const int32_t got = token_or_last((int32_t)first, (uint32_t)(t - first), end);
+          EXPECT(got == (t < end ? t : end - 1), "token %lld of %d: %d", (long long)t, end, got);
+          EXPECT(tokens_before((int32_t)first, (uint32_t)(t - first), n, end) == (t + n <= end), "tokens %lld+%u of %d",
+                 (long long)t, n, end);
+        }
   if (failures) {
     fprintf(stderr, "%d failures\n", failures);
     return 1;

@@ -276,6 +276,20 @@ inline int32_t dims_workers(int32_t dv, int32_t dtype, int32_t heads, int32_t cu
   const int64_t resident = (int64_t)cus * (dtype == TMLA_FP32 && dv <= 256 ? 2 : 1);
   return (int32_t)(resident / gy > 0 ? resident / gy : 1);
 }
+// Lengths of a generic call are cut to the cache's capacity and to this, so
+// that a token index up to 128 past a sequence's end stays below 2^31.
+constexpr int32_t kMaxGenericLen = INT32_MAX - 128;
+// Token `ahead` tokens after `first`, or the last one before `end`; and
+// whether the `n` tokens from it on all lie before `end`. In unsigned
+// arithmetic: the copies of mla_decode_dims.hip run up to three 64-token steps
+// past the end (first + ahead < 2^32).
+constexpr int32_t token_or_last(int32_t first, uint32_t ahead, int32_t end) {
+  const uint32_t t = (uint32_t)first + ahead;
+  return t < (uint32_t)end ? (int32_t)t : end - 1;
+}
+constexpr bool tokens_before(int32_t first, uint32_t ahead, uint32_t n, int32_t end) {
+  return (uint32_t)first + ahead + n <= (uint32_t)end;
+}
 constexpr int64_t kDimsMaxGrid = 1 << 22;  // workgroups along x (512 threads each)
 
 // Workspace of a generic call: the float32 partial rows, then their lse

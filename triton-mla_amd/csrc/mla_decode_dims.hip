@@ -260,7 +260,7 @@ __device__ __forceinline__ void dims_body(const DimsArgs& a, bool paged) {
     auto v_row = [&]() __attribute__((always_inline)) { return 8 * hw + (lane_id_fresh() >> 3); };
     auto r_row = [&]() __attribute__((always_inline)) { return 8 * hw + ((lane_id_fresh() / NP) & 7); };
     auto tok_of = [&](int st, int row) __attribute__((always_inline)) {
-      return min(tok0 + (st * C::TW + tw) * kSub + row, end - 1);
+      return token_or_last(tok0, ((uint32_t)st * C::TW + tw) * kSub + row, end);
     };
     auto raw_page = [&](int t) __attribute__((always_inline)) { return paged ? bt_row[page_slot_of(a, t)] : 0; };
     // Table entries of step st: the sub-tile's one page where a page holds
@@ -284,10 +284,11 @@ __device__ __forceinline__ void dims_body(const DimsArgs& a, bool paged) {
       const int rr = 8 * hw + ((ln / NP) & 7);
       const int v_piece = ((ln & 7) ^ piece_swizzle(ln >> 3, hw)) * 16;
       const int r_piece = DV * 2 + ((ln % NP) ^ ((rr / (16 / NP)) & (NP - 1))) * 16;
-      const int t0 = tok0 + (st * C::TW + tw) * kSub;
+      const uint32_t ahead = ((uint32_t)st * C::TW + tw) * kSub;
       const char *src, *rsrc;
-      if (a.uni && t0 + kSub <= end) {
+      if (a.uni && tokens_before(tok0, ahead, kSub, end)) {
         // one scalar base and 32-bit lane offsets
+        const int t0 = tok0 + ahead;
         const char* row0 = a.kv + row_off(a, paged, b, t0, __builtin_amdgcn_readfirstlane(pg.v));
         src = row0 + (uint32_t)((8 * hw + (ln >> 3)) * (uint32_t)a.kv_s1 + v_piece);
         rsrc = row0 + (uint32_t)(rr * (uint32_t)a.kv_s1 + r_piece);
@@ -622,6 +623,8 @@ __global__ __launch_bounds__(256) void mla_dims_f32_kernel(DimsArgs a) {
     const int slices = (end - tok0 + 15) / 16;
     const int32_t* bt_row = paged ? a.bt + (int64_t)b * a.bt_sb : nullptr;
 
+    // (RING slices of 16 tokens past the end: within what kMaxGenericLen leaves)
+    static_assert((C::RING + 2) * 16 <= INT32_MAX - kMaxGenericLen, "look-ahead");
     auto tok_of = [&](int sl, int row) __attribute__((always_inline)) { return min(tok0 + sl * 16 + row, end - 1); };
     // raw table entry of the slice's one page (a.uni: pages of whole slices),
     // else of row 4 * wave + lane % 4 of slice sl

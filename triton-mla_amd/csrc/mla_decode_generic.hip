@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void mla_generic_partial_kernel(GenericArgs a)
 
   // (lengths cut to the capacity, and far enough below 2^31 that n0 + tile
   // cannot wrap)
-  const int n = (int)min(min((int64_t)max(a.seqlens[b], 0), a.capacity), (int64_t)INT32_MAX - 128);
+  const int n = (int)min(min((int64_t)max(a.seqlens[b], 0), a.capacity), (int64_t)kMaxGenericLen);
   const int split_len = (int)(((int64_t)n + a.splits - 1) / a.splits);
   const int start = (int)min((int64_t)s * split_len, (int64_t)n);
   const int end = (int)min((int64_t)start + split_len, (int64_t)n);
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(256) void mla_generic_mfma_kernel(GenericArgs a) {
   char* const Pw = VT + DV * kMP + wave * 16 * kMP;    // [16 heads][kMP] of this wave
   char* const Qw = VT + DV * kMP + 4 * 16 * kMP + wave * 16 * rp;  // [16 heads][rp] of this wave
 
-  const int n = (int)min(min((int64_t)max(a.seqlens[b], 0), a.capacity), (int64_t)INT32_MAX - 128);
+  const int n = (int)min(min((int64_t)max(a.seqlens[b], 0), a.capacity), (int64_t)kMaxGenericLen);
   const int split_len = (int)(((int64_t)n + a.splits - 1) / a.splits);
   const int start = (int)min((int64_t)s * split_len, (int64_t)n);
   const int end = (int)min((int64_t)start + split_len, (int64_t)n);
@@ -790,7 +790,7 @@ static int generic_call(const void* q, int64_t q_stride_b, int64_t q_stride_h, c
     d.out_sb = out_stride_b;
     d.out_sh = out_stride_h;
     d.lse = lse;
-    d.len_cap = (int32_t)(a.capacity < INT32_MAX - 128 ? a.capacity : INT32_MAX - 128);
+    d.len_cap = (int32_t)(a.capacity < kMaxGenericLen ? a.capacity : kMaxGenericLen);
     d.uni = (!paged || page_size % (dtype == TMLA_FP32 ? 16 : 32) == 0) && d.kv_s1 > 0 && d.kv_s1 < (1 << 26) ? 1 : 0;
     d.part = a.mid_o;
     d.part_lse = a.mid_lse;
