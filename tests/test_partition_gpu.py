@@ -126,3 +126,32 @@ def test_ranges_across_many_sequences(gpu, heads):
     torch.testing.assert_close(out.float().cpu(), torch.from_numpy(ref_out), **OUT_TOL)
     torch.testing.assert_close(lse.cpu()[valid], torch.from_numpy(ref_lse)[valid], **LSE_TOL)
     assert torch.all(out.cpu()[~valid] == 0) and torch.all(torch.isneginf(lse.cpu()[~valid]))
+
+
+@pytest.mark.parametrize("batch,workers", [(64, 256), (65, 256), (300, 800), (300, 64), (600, 256)])
+def test_combine_slots_of_many_sequences(gpu, batch, workers):
+    """The combine's walk over the lengths: one sequence per lane (64), the four
+    waves sharing it (65), several sequences per thread (300, 600), snapped and
+    straddling. Against the oracle, and bit for bit against the single launch,
+    which finds its slots in the partial kernel's own walk, where it applies."""
+    from triton_mla.kernel import DecodeLaunch
+
+    heads = 16
+    g = torch.Generator().manual_seed(batch + workers)
+    lens = torch.randint(0, 500, (batch,), generator=g, dtype=torch.int32)
+    lens[[0, batch - 1]] = torch.tensor([0, 449], dtype=torch.int32)
+    q = torch.randn(batch, heads, D_LATENT + D_ROPE, generator=g).to(torch.bfloat16)
+    kv = torch.randn(batch * 8, TILE, D_LATENT + D_ROPE, generator=g).to(torch.bfloat16)
+    bt = torch.randperm(batch * 8, generator=g).view(batch, 8).int()
+    print(f"combine slots batch={batch} workers={workers} pieces={pieces(lens.tolist(), workers)}", flush=True)
+    call = DecodeLaunch(q.to(gpu), kv.to(gpu), lens.to(gpu), bt.to(gpu), D_LATENT, SCALE, None, workers)
+    out, lse = call.run()
+    out, lse = out.clone(), lse.clone()
+    out1, lse1 = call.run(single_launch=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out, out1) and torch.equal(lse, lse1)
+    ref_out, ref_lse = oracle.mla_decode_ref(bits(q), bits(kv), lens.numpy(), bt.numpy(), D_LATENT, SCALE)
+    valid = lens > 0
+    torch.testing.assert_close(out.float().cpu(), torch.from_numpy(ref_out), **OUT_TOL)
+    torch.testing.assert_close(lse.cpu()[valid], torch.from_numpy(ref_lse)[valid], **LSE_TOL)
+    assert torch.all(out.cpu()[~valid] == 0) and torch.all(torch.isneginf(lse.cpu()[~valid]))
