@@ -54,3 +54,20 @@ def test_other_dims_through_the_cli(gpu, tmp_path, dims, dtype):
         assert str(int(r[k])) == r[k], (k, r[k])
     assert f"generic-{dims[0]}+{dims[1]}" in r["config"]
     assert float(r["triton_us"]) > 0 and float(r["eager_us"]) > 0
+
+
+@pytest.mark.parametrize("dims,config,splits", [(("256", "32"), "hip/balanced256/generic-256+32", 16),
+                                                (("32", "16"), "hip/splits4/generic-32+16", 4)])
+def test_other_dims_run_the_public_default(gpu, tmp_path, dims, config, splits):
+    """--splits balanced (the default) times what mla_decode runs by itself: the
+    balanced partition where the kernels of the usual dims take the call (16
+    tiles a sequence, a worker each, 256 compute units), uniform pieces
+    elsewhere."""
+    path = tmp_path / "bench.csv"
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "triton-mla_amd"))
+    args = ["--batch", "2", "--seqlen", "1000", "--heads", "16", "--no-compile", "--no-eager", "--reps", "5",
+            "--head-dim-v", dims[0], "--rope-dim", dims[1], "--csv", str(path)]
+    print("triton-mla-bench " + " ".join(args), flush=True)
+    subprocess.run([sys.executable, "-m", "triton_mla.bench"] + args, check=True, env=env, timeout=300)
+    r = list(csv.DictReader(open(path)))[0]
+    assert r["config"] == config and int(r["num_splits"]) == splits

@@ -70,13 +70,16 @@ def bench_one(inp, args, device, flush, compiled, writer, gpu):
     if generic:
         if args.kv_fp8 != "none":
             raise SystemExit("--kv-fp8 runs at --head-dim-v 512 --rope-dim 64 only")
-        if splits is None:
+        # the public call's default: the balanced partition, or uniform pieces
+        # where its kernels do not take the call
+        workers = kernel_mod._generic_workers(inp.q, inp.kv_cache, inp.head_dim_v) if splits is None else 0
+        if splits is None and workers == 0:
             splits = kernel_mod._generic_splits(inp.batch, inp.heads, inp.kv_cache.shape[1] * inp.block_table.shape[1],
                                                 _num_sms(device),
                                                 max(_native.load().tmla_generic_heads_per_workgroup(
                                                     inp.head_dim_v, inp.q.shape[-1] - inp.head_dim_v,
                                                     _native.DTYPE_CODE[inp.q.dtype]), 1))
-        call = _GenericCall(inp, splits)
+        call = _GenericCall(inp, splits, workers)
     elif args.kv_fp8 != "none":
         # the HIP decode reads the E4M3 cache; the PyTorch baselines decode the
         # same values dequantised to the input dtype
@@ -147,8 +150,8 @@ class _GenericCall:
     """A decode at other head dims or fp32 (the generic kernels through the
     public mla_decode), with DecodeLaunch's run/out/workers/splits."""
 
-    def __init__(self, inp, splits):
-        self.inp, self.splits, self.workers = inp, splits, 0
+    def __init__(self, inp, splits, workers):
+        self.inp, self.splits, self.workers = inp, splits, workers
         self.out = None
 
     def run(self):

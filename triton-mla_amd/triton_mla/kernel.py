@@ -482,6 +482,17 @@ def _generic_splits(batch, num_heads, capacity, num_sms, heads_per_wg=16):
     return max(1, min(by_cus, by_len, 65535))
 
 
+def _generic_workers(q, kv_cache, head_dim_v):
+    """Workers of the balanced partition a generic call (3-D q and cache)
+    runs with num_splits=None, where its kernels take the call: the usual
+    dims, rows on 16-byte boundaries. 0: uniform pieces."""
+    elems = 16 // q.element_size()
+    if not (_aligned(q, elems) and _aligned(kv_cache, elems)):
+        return 0
+    return _native.load().tmla_generic_workers(head_dim_v, q.shape[-1] - head_dim_v, _native.DTYPE_CODE[q.dtype],
+                                               q.shape[1], _num_sms(q.device))
+
+
 def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax_scale, num_splits, return_lse,
                     learn=None):
     """``mla_decode`` at head dims or an element type the matrix-core kernels
@@ -538,11 +549,7 @@ def _generic_decode(q, kv_cache, cache_seqlens, block_table, head_dim_v, softmax
     dtype = _native.DTYPE_CODE[q.dtype]
     workers = 0
     if num_splits is None:
-        # the balanced partition where its kernels take the call (the usual
-        # dims, rows on 16-byte boundaries), uniform pieces otherwise
-        elems = 16 // q.element_size()
-        if _aligned(q, elems) and _aligned(kv_cache, elems):
-            workers = lib.tmla_generic_workers(head_dim_v, d_rope, dtype, num_heads, _num_sms(device))
+        workers = _generic_workers(q, kv_cache, head_dim_v)
         if workers == 0:
             per_wg = lib.tmla_generic_heads_per_workgroup(head_dim_v, d_rope, dtype)
             num_splits = _generic_splits(batch, num_heads, capacity, _num_sms(device), max(per_wg, 1))
