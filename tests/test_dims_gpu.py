@@ -1,6 +1,7 @@
 """The matrix-core kernels of other head dims and float32 (mla_decode_dims.hip):
 head_dim_v 64 to 512 and rope_dim 16 to 64 with 16-byte aligned rows, balanced
-(num_splits=None) and uniform (float32 with a split count keeps the general
+(num_splits=None: here one tile a worker; straddling ranges and longer pieces
+with given worker counts) and uniform (float32 with a split count keeps the general
 form, checked all the same), against the float64 oracle and, through the
 C ABI, against the general forms that the same call takes when its output
 rows are not 16-byte aligned.
@@ -72,6 +73,68 @@ def test_dims_match_oracle(gpu, dv, dr, dtype, heads, page, splits):
                               softmax_scale=scale, num_splits=splits, return_lse=True)
         torch.cuda.synchronize()
         _check(out, lse, q, kv, lens, bt, dv, scale, dtype)
+
+
+def _balanced(lib, gpu, q, kv, lens, bt, dv, dr, scale, workers):
+    """tmla_mla_decode_generic_balanced with a given worker count."""
+    from triton_mla import _native
+
+    batch, heads, dtype = q.shape[0], q.shape[1], q.dtype
+    gq, gkv, gl, gbt = q.to(gpu), kv.to(gpu), lens.to(gpu), None if bt is None else bt.to(gpu)
+    out = torch.full((batch, heads, dv), 7.0, dtype=dtype, device=gpu)
+    lse = torch.full((batch, heads), 7.0, device=gpu)
+    ws = torch.empty(lib.tmla_generic_balanced_workspace_bytes(batch, heads, dv, workers), dtype=torch.uint8, device=gpu)
+    _native.check(lib.tmla_mla_decode_generic_balanced(
+        gq.data_ptr(), gq.stride(0), gq.stride(1), gkv.data_ptr(), gkv.stride(0), gkv.stride(1),
+        gkv.shape[1] if bt is None else gkv.shape[0], 1 if bt is None else gkv.shape[1],
+        None if bt is None else gbt.data_ptr(), 0 if bt is None else gbt.stride(0), 1 if bt is None else gbt.shape[1],
+        gl.data_ptr(), batch, heads, dv, dr, _native.DTYPE_CODE[dtype], scale, workers, out.data_ptr(), out.stride(0),
+        out.stride(1), lse.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream), "balanced")
+    torch.cuda.synchronize()
+    return out, lse
+
+
+# every kernel class (16 bits up to 256 dims and at 512, float32 with 16 and
+# 32 heads a workgroup), a dense cache, pages of whole sub-tiles and smaller
+SEGMENT_CASES = [
+    (64, 16, HF, 33, 0), (128, 64, BF, 130, 16), (256, 32, BF, 128, 64), (256, 64, HF, 20, 48), (512, 32, BF, 64, 32),
+    (512, 16, HF, 129, 0), (512, 64, F32, 16, 64), (256, 32, F32, 40, 16), (64, 16, F32, 33, 0),
+]
+
+
+@pytest.mark.parametrize("workers,snapped", [(5, False), (1, False), (30, True)])
+@pytest.mark.parametrize("dv,dr,dtype,heads,page", SEGMENT_CASES)
+def test_dims_ranges_across_sequences(gpu, dv, dr, dtype, heads, page, workers, snapped):
+    """Ranges over several sequences (the next segment reuses the ring, Q and
+    the merge area in LDS, and starts mid-range on the partition's line), empty
+    ones between them, and snapped pieces of several tiles."""
+    from triton_mla import _native
+
+    q, kv, lens, bt = _inputs(dv, dr, dtype, heads, page, 3 * dv + heads)
+    tiles = [-(-n // 64) for n in lens.tolist()]
+    chunk = -(-sum(tiles) // workers)
+    assert chunk > 1 and (sum(-(-t // chunk) for t in tiles) <= workers) == snapped
+    print(f"segments {dv}+{dr} {NAME[dtype]} heads={heads} page={page} workers={workers}", flush=True)
+    out, lse = _balanced(_native.load(), gpu, q, kv, lens, bt, dv, dr, 0.2, workers)
+    _check(out, lse, q, kv, lens, bt, dv, 0.2, dtype)
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_dims_many_sequences(gpu, dtype):
+    """More than 64 sequences (each lane of the partition takes several):
+    snapped and straddling ranges."""
+    from triton_mla import _native
+
+    g = torch.Generator().manual_seed(21)
+    dv, dr, heads, batch = 128, 32, 17, 150
+    lens = torch.randint(0, 300, (batch,), generator=g, dtype=torch.int32)
+    lens[[1, 3, 70]] = torch.tensor([1, 0, 64], dtype=torch.int32)
+    q = torch.randn(batch, heads, dv + dr, generator=g).to(dtype)
+    kv, bt = _paged(torch.randn(batch, 300, dv + dr, generator=g).to(dtype), 64, g)
+    for workers in (600, 40):
+        print(f"150 sequences {NAME[dtype]} workers={workers}", flush=True)
+        out, lse = _balanced(_native.load(), gpu, q, kv, lens, bt, dv, dr, 0.2, workers)
+        _check(out, lse, q, kv, lens, bt, dv, 0.2, dtype)
 
 
 @pytest.mark.parametrize("dtype", [BF, F32])
