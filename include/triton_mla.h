@@ -267,7 +267,10 @@ int tmla_mla_decode_causal(const void* q, int64_t q_stride_b, int64_t q_stride_h
  * (scale_stride_1 = 0) and pages of a power-of-two multiple of 32 tokens, the
  * cache is widened once per workgroup into the 16-bit kernel's ring; other
  * calls run groups of 16 heads that each stream the cache.
+ * tmla_fp8_heads_per_workgroup tells which: 128 (the most heads that share a
+ * widened cache) or 16.
  */
+int32_t tmla_fp8_heads_per_workgroup(int32_t num_heads, int32_t paged, int32_t page_size, int64_t scale_stride_1);
 int tmla_mla_decode_fp8(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv,
                         int64_t kv_stride_0, int64_t kv_stride_1, int64_t num_blocks, int32_t page_size,
                         const float* kv_scale, int64_t scale_stride_0, int64_t scale_stride_1,

@@ -154,6 +154,15 @@ def test_generic_workspace_and_rejections(lib):
     assert lib.tmla_generic_heads_per_workgroup(128, 32, 3) == 0
 
 
+def test_fp8_heads_per_workgroup(lib):
+    """The rule by which an fp8 call widens the cache once per workgroup, asked
+    by the host where it shares the workers among the workgroups."""
+    f = lib.tmla_fp8_heads_per_workgroup
+    assert f(17, 1, 64, 0) == 128 and f(128, 1, 32, 0) == 128 and f(1024, 1, 256, 0) == 128
+    for args in ((16, 1, 64, 0), (128, 0, 1, 0), (128, 1, 64, 1), (128, 1, 16, 0), (128, 1, 96, 0), (128, 1, 0, 0)):
+        assert f(*args) == 16, args
+
+
 def test_generic_balanced_workers_and_rejections(lib):
     """The balanced generic call: its worker counts (one resident workgroup
     per compute unit; two in float32 up to 256 dims; shared along the heads),

@@ -156,6 +156,19 @@ inline LaunchPlan plan_launch_g16(int32_t batch, int32_t num_heads, int32_t num_
   return p;
 }
 
+// fp8 cache: up to this many heads the 16-head-group kernel runs (its
+// workgroups stream the cache on their own); above, where pages are a power of
+// two of whole 32-token sub-tiles with one scale each (or for the cache), the
+// 16-bit kernel with the cache widened once per workgroup into its ring
+#ifndef TMLA_FP8_GROUP_HEADS
+#define TMLA_FP8_GROUP_HEADS 16
+#endif
+constexpr int kFp8GroupHeads = TMLA_FP8_GROUP_HEADS;
+inline bool fp8_ring(int32_t heads, bool paged, int32_t page_size, int64_t scale_s1) {
+  return heads > kFp8GroupHeads && paged && page_size > 0 && page_size % 32 == 0 &&
+         (page_size & (page_size - 1)) == 0 && scale_s1 == 0;
+}
+
 struct Common {
   int32_t batch, heads, dv, dr, dtype, splits, workers;
 };

@@ -103,18 +103,11 @@ constexpr int kHeadsPerWave = 32;   // N of the 32x32x16 MFMA
 #ifndef TMLA_G16_HEADS
 #define TMLA_G16_HEADS 16
 #endif
-// fp8 cache: up to this many heads the 16-head-group kernel runs (its
-// workgroups stream the cache on their own); above, the 16-bit kernel with the
-// cache widened once per workgroup into its ring
-#ifndef TMLA_FP8_GROUP_HEADS
-#define TMLA_FP8_GROUP_HEADS 16
-#endif
 // combine: four heads per wave when one head per wave would take more than
 // this many workgroups
 #ifndef TMLA_COMBINE_WIDE_WGS
 #define TMLA_COMBINE_WIDE_WGS 1024
 #endif
-constexpr int kFp8GroupHeads = TMLA_FP8_GROUP_HEADS;
 constexpr int kG16Heads = TMLA_G16_HEADS;
 constexpr int64_t kCombineWideWgs = TMLA_COMBINE_WIDE_WGS;
 static_assert(kG16Heads <= 16, "one head group per workgroup");
@@ -2293,6 +2286,10 @@ size_t tmla_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim_v
 
 int32_t tmla_partition_segment_tiles(void) { return kSegCostTiles; }
 
+int32_t tmla_fp8_heads_per_workgroup(int32_t num_heads, int32_t paged, int32_t page_size, int64_t scale_stride_1) {
+  return fp8_ring(num_heads, paged != 0, page_size, scale_stride_1) ? 128 : 16;
+}
+
 int tmla_debug_stamps(void* host, size_t bytes) {
 #if TMLA_STAMPS
   const size_t n = sizeof(g_stamps) < bytes ? sizeof(g_stamps) : bytes;
@@ -2396,16 +2393,15 @@ int decode_launch(const void* q, int64_t q_stride_b, int64_t q_stride_h, const v
   // power-of-two page size: page slots and in-page rows by shifts and masks
   const bool uni = paged && (page_size % kSubTokens == 0) && a.page_shift >= 0;
   if (f8) {
-    // fp8 cache, always two launches (no in-kernel merge). More than
-    // kFp8GroupHeads heads with one scale per page (or per tensor) and pages
-    // of whole sub-tiles: the 16-bit kernel with the cache widened once per
-    // workgroup into its ring; otherwise groups of 16 heads, each streaming
-    // and widening the cache on its own.
+    // fp8 cache, always two launches (no in-kernel merge): the 16-bit kernel
+    // with the cache widened once per workgroup into its ring, or groups of 16
+    // heads, each streaming and widening the cache on its own (fp8_ring).
     a.kv_scale = f8->scale;
     a.sc_s0 = f8->s0;
     a.sc_s1 = f8->s1;
     hipError_t e;
-    if (uni && f8->s1 == 0 && num_heads > kFp8GroupHeads) {
+    static_assert(kSubTokens == 32, "fp8_ring's pages of whole sub-tiles");
+    if (fp8_ring(num_heads, paged, page_size, f8->s1)) {
       const LaunchPlan plan = plan_launch(batch, num_heads, num_splits, num_workers, cap_tokens, mid_o_bytes,
                                           mode == 0 ? 0 : 2, current_cu_count());
       a.fused = 0;

@@ -59,6 +59,7 @@ SIGNATURES = {
     "tmla_mla_decode_generic": (ctypes.c_int, [
         _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _vp, _i64, _i32, _vp, _i32, _i32, _i32, _i32, _i32, _f32,
         _i32, _vp, _i64, _i64, _vp, _vp, _sz, _vp]),
+    "tmla_fp8_heads_per_workgroup": (_i32, [_i32, _i32, _i32, _i64]),
     "tmla_generic_workers": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "tmla_generic_balanced_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
     "tmla_mla_decode_generic_balanced": (ctypes.c_int, [

@@ -111,10 +111,15 @@ def _balanced_workers(num_sms: int, heads: int, heads_per_workgroup: int, tiles:
     workgroups a worker's range takes along the (virtual) heads, since each
     round of workgroups pays its start-up, its finalize and its partials
     again (16 sequences of 1K to 8K tokens, two query tokens of 128 heads:
-    79 us with 256 workers in two rounds, 59 us with 128 in one).
+    79 us with 256 workers in two rounds, 59 us with 128 in one). Measured
+    at 0.25 to 16 tiles per compute unit, 2 to 88 groups, 16-bit and fp8
+    caches: 1.0 to 6.1 times the speed of one worker per compute unit
+    throughout (profiles/mla_decode_shared_workers.md), also below the line
+    drawn here and where the groups leave compute units idle (88 groups: 176
+    of 256; two or four rounds take 0.8 of that time there).
     Calls whose cache holds fewer than four 64-token tiles per compute unit
-    keep one worker per compute unit, the partition (and so the bits) of a
-    single-token call."""
+    keep one worker per compute unit all the same: the partition, and so the
+    bits, of a single-token call, which their callers compare them with."""
     groups = _cdiv(heads, heads_per_workgroup)
     if groups == 1 or tiles < 4 * num_sms:
         return num_sms
@@ -285,12 +290,9 @@ class DecodeLaunch:
             if num_workers:
                 self.workers = int(num_workers)
             else:
-                # heads per workgroup: 128, or 16 for an fp8 cache whose pages
-                # are not widened into the 16-bit ring
-                ring = not fp8 or (scale_args[2] == 0 and block_table is not None and page_size % 32 == 0
-                                   and page_size & (page_size - 1) == 0)
-                self.workers = _balanced_workers(_num_sms(device), vheads, 128 if ring else 16,
-                                                 batch * _cdiv(capacity, 64))
+                per_wg = 128 if not fp8 else self.lib.tmla_fp8_heads_per_workgroup(
+                    vheads, int(block_table is not None), page_size, scale_args[2])
+                self.workers = _balanced_workers(_num_sms(device), vheads, per_wg, batch * _cdiv(capacity, 64))
         dev_idx = device.index if device.index is not None else torch.cuda.current_device()
         self._dev_idx = dev_idx
         # The library's answers for this shape (workspace size, the counter
