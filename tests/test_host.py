@@ -244,3 +244,27 @@ def test_kept_arguments_refuse_what_the_full_path_refuses(monkeypatch):
     assert K._fast_call_other(q, kv, lens, None, 256.0, None, None, None) is None
     with pytest.raises(AttributeError):  # the full path's refusal
         K.mla_decode(q, kv, lens, head_dim_v=256.0)
+
+
+@pytest.mark.parametrize("what", ["lens", "table", "one token", "scale"])
+def test_calls_that_cannot_be_kept_are_not_looked_up(monkeypatch, what):
+    """int64 lengths or tables (converted on each call), one query token in four
+    dims over a 16-bit cache and a number as the fp8 scale always take the full
+    path: no key is built and nothing is learned for them."""
+    from triton_mla import kernel as K
+
+    def learned(*args):
+        raise AssertionError("learned")
+
+    q, kv, lens = torch.zeros(2, 16, 576), torch.zeros(2, 64, 576), torch.tensor([40, 20], dtype=torch.int32)
+    bt, scale = torch.zeros(2, 1, dtype=torch.int32), None
+    if what == "lens":
+        lens = lens.long()
+    elif what == "table":
+        bt = bt.long()
+    elif what == "one token":
+        q = q.unsqueeze(1)
+    else:
+        kv, scale = kv.to(torch.uint8), 0.5
+    monkeypatch.setattr(K, "_learn_other", learned)
+    assert K._fast_call_other(q, kv, lens, bt, 512, None, None, scale) is None

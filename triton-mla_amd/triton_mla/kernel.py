@@ -738,6 +738,12 @@ def _fast_call_other(q, kv_cache, cache_seqlens, block_table, head_dim_v, softma
     take 14 to 15.5 us). The workspace is the stream's (see _STREAM_WS): these entries'
     kernels too write every workspace byte they read."""
     try:
+        # calls that are never kept: their key costs 1 to 2 us
+        if (cache_seqlens.dtype is not torch.int32
+                or (block_table is not None and block_table.dtype is not torch.int32)
+                or (kv_scale is None and q.dim() == 4 and q.shape[1] == 1)
+                or (kv_scale is not None and type(kv_scale) is not torch.Tensor)):
+            return None
         key = (q.shape, q.stride(), q.dtype, q.get_device(), kv_cache.shape, kv_cache.stride(), kv_cache.dtype,
                kv_cache.get_device(), cache_seqlens.dtype, cache_seqlens.get_device(), cache_seqlens.shape,
                cache_seqlens.stride(),
