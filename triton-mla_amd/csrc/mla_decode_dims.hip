@@ -408,7 +408,12 @@ __device__ __forceinline__ void dims_body(const DimsArgs& a, bool paged) {
         }
         if constexpr (j == NKC - 1) {
           // online softmax, base 2, with the lazy rescale: lane holds head
-          // lane%32, tokens 8 (r / 4) + 4 hi + r % 4 in register r
+          // lane%32, tokens 8 (r / 4) + 4 hi + r % 4 in register r. (A
+          // reference that follows every new max leaves that token's
+          // probability exact: error against float64 1.728e-3 instead of
+          // 1.752e-3 at 32 sequences, 256 + 32 in bf16, 1.76e-3 instead of
+          // 1.81e-3 at 512 + 32; it takes 68.7 us instead of 61 and 61.5
+          // instead of 50.7. v_exp_f32 and exp2f give the same error.)
           s_fence(s);
           if (base + kSub > end) {
 #pragma unroll
