@@ -95,13 +95,13 @@ def test_mfma_result_scan_follows_branches(tmp_path):
     assert build.mfma_result_hazards(_asm(tmp_path, agpr + read)) == []
 
 
-def test_mfma_operand_scan(tmp_path):
+def test_operand_scan(tmp_path):
     mfma = _in_asm("\tv_mfma_f32_32x32x16_bf16 v[2:17], v[222:225], v[22:25], v[2:17]\n")
     back = "\tv_accvgpr_read_b32 v24, a132\n"
     other = "\tv_add_u32_e32 v100, v101, v102\n"
 
     def hits(body):
-        return len(build.mfma_operand_hazards(_asm(tmp_path, body + "\ts_endpgm\n")))
+        return len(build.operand_hazards(_asm(tmp_path, body + "\ts_endpgm\n")))
 
     # an operand brought back from an AGPR right before, or one instruction before
     assert hits(back + mfma) == 1 and hits(back + other + mfma) == 1
@@ -114,6 +114,13 @@ def test_mfma_operand_scan(tmp_path):
     assert hits(back + mfma.replace("\t;;#ASMSTART\n", "")) == 0
     # before a branch, and in one of two predecessors
     assert hits(back + "\ts_cbranch_scc0 .LBB0_1\n" + other + ".LBB0_1:\n" + mfma) == 1
+    # ... but not after a write in inline asm, which it does not see either
+    own = mfma.replace("\t;;#ASMSTART\n", "")
+    assert hits(_in_asm("\tv_accvgpr_read_b32 v24, a132\n") + own) == 1
+    dpp = "\tv_add_u32_dpp v60, v61, v60 row_shr:1 row_mask:0xf bank_mask:0xf\n"
+    swap = _in_asm("\tv_permlane16_swap_b32 v61, v62\n")
+    assert hits(swap + dpp) == 1 and hits(swap + other + other + dpp) == 0
+    assert hits("\tv_mov_b32_e32 v61, 0\n" + dpp) == 0
     # both registers of a swap are written
     assert hits("\tv_permlane32_swap_b32 v60, v223\n" + mfma) == 1
 
@@ -182,5 +189,5 @@ __global__ void k(const i16x8* a, const i16x8* b, f32x16* o, short x) {
                                                         str(src), "-o", str(out)], check=True, capture_output=True)
         assert any(ins.asm and ins.op.startswith("v_mfma") for _, blocks in asm_checks.kernels(str(out))
                    for blk in blocks for ins in blk.ins)
-        found.append(len(asm_checks.mfma_operand_hazards(str(out))))
+        found.append(len(asm_checks.operand_hazards(str(out))))
     assert found[0] > 0 and found[1] == 0

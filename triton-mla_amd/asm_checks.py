@@ -10,9 +10,9 @@ of one build:
     that covers it (LDS operations return in order, so ``lgkmcnt(n)`` covers
     all but the newest n; scalar loads return in any order and are covered by
     ``lgkmcnt(0)`` only);
-  * ``mfma_operand_hazards``: a vector-ALU instruction (a copy out of an AGPR
-    for instance) writes an operand of an inline-asm MFMA fewer than two wait
-    states before it;
+  * ``operand_hazards``: a vector-ALU instruction (a copy out of an AGPR for
+    instance) writes an operand of an MFMA or of a DPP move fewer than two wait
+    states before it, where one of the two is inline asm;
   * ``mfma_result_touches``: the result of an MFMA is read or overwritten
     before the MFMA has finished, where one of the two is inline asm.
 
@@ -27,7 +27,7 @@ from __future__ import annotations
 import re
 from typing import NamedTuple
 
-OPERAND_WAIT_STATES = 2  # vector-ALU write of a register -> MFMA that reads it
+OPERAND_WAIT_STATES = 2  # vector-ALU write of a register -> MFMA or DPP move that reads it
 RESULT_WINDOW = 18       # wait states after which any MFMA used here has finished
 _COUNTER = 15            # lgkmcnt counts to 15
 
@@ -202,18 +202,21 @@ def inflight_touches(asm_path: str) -> list:
     return _scan(asm_path, _asm_load, step, min)
 
 
-def _asm_mfma(ins: Ins) -> bool:
-    return ins.asm and ins.op.startswith("v_mfma")
+def _early_reader(ins: Ins) -> bool:
+    return ins.op.startswith("v_mfma") or ins.op.endswith("_dpp")
 
 
-def mfma_operand_hazards(asm_path: str) -> list:
-    """(writer, MFMA) pairs: see the module's docstring."""
+def operand_hazards(asm_path: str) -> list:
+    """(writer, MFMA or DPP move) pairs: see the module's docstring."""
 
     # register -> (wait states since a vector-ALU instruction wrote it, that instruction)
     def step(state, ins, report):
-        if _asm_mfma(ins):
-            for reg in frozenset().union(*ins.parts[1:4]) & state.keys():
-                report(ins, state[reg][1])
+        if state and _early_reader(ins):
+            # (the first operand is the result; a DPP move may keep old lanes of it)
+            read = ins.parts[1:4] if ins.op.startswith("v_mfma") else ins.parts
+            for reg in frozenset().union(*read) & state.keys():
+                if ins.asm or state[reg][1].asm:
+                    report(ins, state[reg][1])
         for reg, (since, writer) in list(state.items()):
             if since + ins.nop >= OPERAND_WAIT_STATES:
                 del state[reg]
@@ -225,7 +228,7 @@ def mfma_operand_hazards(asm_path: str) -> list:
                 if reg[0] != "s":
                     state[reg] = (0, ins)
 
-    return _scan(asm_path, _asm_mfma, step, min)
+    return _scan(asm_path, lambda ins: ins.asm and ins.op.startswith("v_"), step, min)
 
 
 def mfma_result_hazards(asm_path: str, window: int = RESULT_WINDOW) -> list:

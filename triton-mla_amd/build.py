@@ -30,7 +30,7 @@ import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
-from asm_checks import inflight_touches, mfma_operand_hazards, mfma_result_hazards
+from asm_checks import inflight_touches, mfma_result_hazards, operand_hazards
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -63,7 +63,7 @@ SCRATCH_ALLOWANCE = {
 ASM_CHECKS = {
     "an inline-asm load's destination touched before it has arrived": inflight_touches,
     "an inline-asm MFMA result touched before it is ready": mfma_result_hazards,
-    "an inline-asm MFMA operand written too shortly before it": mfma_operand_hazards,
+    "an operand of an MFMA or DPP move written too shortly before it": operand_hazards,
 }
 
 
